@@ -16,7 +16,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
-SOURCES = ["rollout.hip", "memory.hip", "ppo.hip", "large.hip", "fixtures.hip", "fixed_ppo.hip", "capi.hip"]
+SOURCES = ["rollout.hip", "rollout_small.hip", "memory.hip", "ppo.hip", "large.hip", "fixtures.hip", "fixed_ppo.hip", "capi.hip"]
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off", "-fno-fast-math",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-I" + os.path.join(ROOT, "include"), "-I" + os.path.join(HERE, "csrc")]

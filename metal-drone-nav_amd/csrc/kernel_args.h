@@ -79,7 +79,11 @@ struct RolloutArgs {
     // env's active level [N] (null: no bank, rows get MDN_BANK_REHEARSAL)
     const uint32_t* bank_active;
     uint32_t* bank_transition;
+    uint32_t epw;          // envs per wavefront of the small-fleet instances (set by their launcher)
 };
+// Most envs that the small-fleet instances take: four per wavefront, four
+// wavefronts per CU.
+constexpr uint32_t SMALL_FLEET = 4096;
 // Per-episode work after a reset (rollout.hip episode_kernel): the
 // episode's plant and hover rpm (sim.metal:62-81) and its navigation task
 // (sim.metal:122-141), for every env (first) or the envs whose episode
@@ -193,6 +197,10 @@ hipError_t nav_launch_reset(const nav::RolloutArgs* a, hipStream_t stream);
 hipError_t nav_launch_episode(const nav::EpisodeArgs* a, hipStream_t stream);
 hipError_t nav_launch_rollout(const nav::RolloutArgs* a, int lanes_per_env, int ring_slots, uint32_t actor_obs,
                               hipStream_t stream);
+// the small-fleet instances (8 lanes per env; rollout_small.hip), which
+// nav_launch_rollout chooses
+hipError_t nav_launch_rollout_small(const nav::RolloutArgs* args, int ring_slots, uint32_t actor_obs,
+                                    hipStream_t stream);
 hipError_t nav_launch_memory_hint(const nav::MemoryArgs* a, hipStream_t stream);
 hipError_t nav_launch_validate(const MdnTaskState* tasks, const MdnPhysicsParams* phys, uint32_t n, uint32_t* out,
                                hipStream_t stream);

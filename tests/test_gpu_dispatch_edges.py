@@ -1,0 +1,62 @@
+"""The sizes at which a kernel or its split of the work changes, against the
+oracle at tolerance 0: fleets around the small-fleet rollout's envs per
+wavefront (1,024 envs each) and its limit (4,096), with every ring size, the
+guided actor and per-episode plants."""
+import sys
+
+import pytest
+
+from gpu_compare import ENV_BUFFERS, ROW_BUFFERS, compare, config, make_pair
+from mdnav import task_runtime, task_settings
+
+pytestmark = pytest.mark.gpu
+
+
+def say(*args):
+    print(*args, flush=True)
+    sys.stdout.flush()
+
+
+def _collect_both(sim, ora, ticks, extra=()):
+    ora.set("actor", sim.get("actor"))
+    ora.set("critic", sim.get("critic"))
+    sim.reset()
+    ora.reset()
+    for count in (ticks, ticks - 1):
+        sim.collect(count)
+        sim.sync()
+        ora.collect(count)
+        bad = compare(sim, ora, ENV_BUFFERS + ROW_BUFFERS + list(extra))
+        assert not bad, bad
+
+
+@pytest.mark.parametrize("n", [1, 3, 5, 1024, 1025, 2048, 2049, 3071, 3073, 4096, 4097])
+def test_fleet_sizes(n):
+    say("case: fleet of", n)
+    sim, _, ora = make_pair(config(n=n, family=1, seed=n, max_steps=3, speed=1.0, distance=3.0), 5)
+    _collect_both(sim, ora, 5)
+
+
+@pytest.mark.parametrize("n", [37, 1030, 4100])
+@pytest.mark.parametrize("delay", [2, 6])
+@pytest.mark.parametrize("obs,memory", [(181, 0), (184, 0), (184, 1)])
+def test_fleet_ring_sizes(n, delay, obs, memory):
+    say("case: fleet of", n, "sensor delay", delay, "inputs", obs, "memory", memory)
+    cfg = config(n=n, family=13, seed=5, max_steps=6, sensor_delay=delay, command_delay=delay, speed=1.5, distance=4.0,
+                 geometry_memory=memory)
+    sim, _, ora = make_pair(cfg, 10, actor_obs=obs)
+    _collect_both(sim, ora, 10)
+
+
+@pytest.mark.parametrize("n,delay,obs", [(1, 0, 184), (1026, 0, 184), (130, 2, 181), (130, 6, 184), (4099, 0, 181)])
+def test_fleet_plants_and_tasks(n, delay, obs):
+    say("case: per-episode plants and tasks, fleet of", n, "sensor delay", delay, "inputs", obs)
+    cfg = config(n=n, family=12, seed=9, sensor_delay=delay, geometry_memory=int(obs == 184), speed=1.5, distance=8.0,
+                 max_steps=400)
+    sim, _, ora = make_pair(cfg, 6, actor_obs=obs)
+    rt, t = task_runtime(1.0), task_settings(2, 12)
+    t["config"]["max_nav_steps"] = 4
+    for x in (sim, ora):
+        x.set_runtime(rt)
+        x.set_tasks(t)
+    _collect_both(sim, ora, 6, ["environment_physics", "task_states"])
