@@ -165,7 +165,7 @@ struct MdnPPO {
     uint32_t updates = 0;
     float *am = nullptr, *av = nullptr, *cm = nullptr, *cv = nullptr;
     // minibatch workspaces: per-chunk partials and the reduced gradient; row
-    // records of the one-chunk path (minibatches of at most 256 rows)
+    // records of minibatches of few chunks (null for larger ones)
     float *part = nullptr, *grad = nullptr, *mb_rec = nullptr;
     double* norm_part = nullptr;
     float* norm_stats = nullptr;
@@ -797,7 +797,7 @@ int mdn_ppo_create(MdnSim* s, uint32_t epochs, uint32_t minibatch, MdnPPO** out)
     guard(dev_alloc(&p->cv, s->shape.critic_count()));
     guard(dev_alloc(&p->part, size_t(chunks) * ppo_partial_stride(s->shape.obs)));
     guard(dev_alloc(&p->grad, ppo_partial_stride(s->shape.obs)));
-    if (M <= ppo::MB_ROWS) guard(dev_alloc(&p->mb_rec, ppo::MB_REC_WORDS));
+    if (chunks <= ppo::MB_MAX_CHUNKS) guard(dev_alloc(&p->mb_rec, size_t(chunks) * ppo::MB_REC_WORDS));
     guard(dev_alloc(&p->norm_part, ppo_normalize_part_words(s->rows())));
     guard(dev_alloc(&p->norm_stats, 2));
     guard(dev_alloc(&p->metric_rows, size_t(p->updates) * 4));
@@ -862,7 +862,6 @@ int ppo_update(MdnPPO* p, uint32_t rollout_index, bool normalize_rows) {
     const std::vector<uint32_t> order = mdn::minibatch_schedule(rows, p->minibatch, p->epochs, rollout_index);
     if (order.size() != p->updates) return fail(MDN_E_STATE, "PPO update count mismatch");
     const size_t first_epoch = order.size() / p->epochs;
-    bool stale_w1t = false;  // transposed first layers behind the flat vectors
     for (size_t u = 0; u < order.size(); u++) {
         const uint32_t begin = order[u];
         const uint32_t b = std::min(p->minibatch, rows - begin);
@@ -880,8 +879,8 @@ int ppo_update(MdnPPO* p, uint32_t rollout_index, bool normalize_rows) {
         ra.actor = s->actor; ra.actor_w1t = s->actor_w1t; ra.critic = s->critic; ra.critic_w1t = s->critic_w1t;
         ra.part = p->part;
         ra.b = b; ra.d = s->shape.obs; ra.clip = 0.2f; ra.vcoef = 0.5f; ra.ecoef = s->cfg.entropy_coef;
-        const bool one_chunk = p->mb_rec && b <= ppo::MB_ROWS;
-        if (one_chunk) {  // one chunk: row and parameter passes over many CUs
+        const bool few = p->mb_rec != nullptr;
+        if (few) {  // few chunks: row and parameter passes over many CUs
             ppo::MbArgs ma;
             ma.r = ra;
             ma.rec = p->mb_rec;
@@ -889,13 +888,10 @@ int ppo_update(MdnPPO* p, uint32_t rollout_index, bool normalize_rows) {
             rc = timed(s, MDN_K_ROWS, [&] { return ppo_launch_minibatch(&ma, s->stream); });
             if (rc) return rc;
         } else {
-            if (stale_w1t) {  // the chunk kernel stages the transposed copies
-                rc = refresh_transposes(s);
-                if (rc) return rc;
-                stale_w1t = false;
-            }
             rc = timed(s, MDN_K_ROWS, [&] { return ppo_launch_rows(&ra, s->stream); });
             if (rc) return rc;
+        }
+        if (!few || b > ppo::CHUNK_ROWS) {
             rc = timed(s, MDN_K_GRADS, [&] {
                 return ppo_launch_grads(p->part, p->grad, b, s->shape.obs, s->stream);
             });
@@ -911,14 +907,13 @@ int ppo_update(MdnPPO* p, uint32_t rollout_index, bool normalize_rows) {
         mdn::adam_corrections(p->optimizer_step, 0.9f, 0.999f, &aa.c1, &aa.c2);
         aa.b = b;
         aa.d = s->shape.obs;
-        // the one-chunk forward stages the flat first layers, so their
+        // the few-chunk forward stages the flat first layers, so their
         // transposed copies are formed once, after the last step
-        aa.keep_w1t = one_chunk ? 0u : 1u;
-        stale_w1t = stale_w1t || one_chunk;
+        aa.keep_w1t = few ? 0u : 1u;
         rc = timed(s, MDN_K_ADAM, [&] { return ppo_launch_adam(&aa, s->stream); });
         if (rc) return rc;
     }
-    if (stale_w1t) {
+    if (p->mb_rec) {  // the rollout reads the transposed first layers
         rc = refresh_transposes(s);
         if (rc) return rc;
     }

@@ -158,15 +158,22 @@ struct RowArgs {
 };
 
 // cpu_reference.hpp:553-567 inputs for one update of both networks.
-// One minibatch of at most 256 rows (a single gradient chunk) split over many
-// workgroups: the row-parallel forward writes per-row records to `rec`, the
-// parameter-parallel pass writes the finished gradient to `grad`.
+// A minibatch of few 256-row gradient chunks split over many workgroups: the
+// row-parallel forward writes per-row records to `rec`, the
+// parameter-parallel pass writes the finished gradient to `grad` (one chunk)
+// or each chunk's partial to r.part.
 struct MbArgs {
     RowArgs r;
-    float* rec;   // [MB_REC_WORDS]: h and delta of actor and critic [4][256][64], row scalars [256][16]
+    float* rec;   // [chunks][MB_REC_WORDS]: h and delta of actor and critic [4][256][64], row scalars [256][16]
     float* grad;  // P_TOTAL: actor, critic, metric sums
 };
-constexpr uint32_t MB_ROWS = 256, MB_REC_WORDS = 4 * 256 * 64 + 256 * 16;
+constexpr uint32_t MB_REC_WORDS = 4 * 256 * 64 + 256 * 16;
+// Most chunks that path takes.  Us per step of one Adam step's kernels, this
+// path and the chunk kernel: 20 and 68 at 2 chunks, 33 and 77 at 16, 65 and
+// 83 at 64, 84 and 85 at 96, 103 and 86 at 128 (its records and their re-reads
+// go through L2, where the chunk kernel keeps them in LDS).
+constexpr uint32_t MB_MAX_CHUNKS = 80;
+constexpr uint32_t CHUNK_ROWS = 256;  // rows of one gradient chunk
 
 struct AdamArgs {
     float* actor; float* critic; float* actor_w1t; float* critic_w1t;

@@ -927,33 +927,57 @@ __global__ __launch_bounds__(CT) void chunk_kernel(RowArgs a) {
     }
 }
 
+// x[0] + x[stride] + ... (n terms) added in order to s, sixteen loads in
+// flight at a time.
+__device__ __forceinline__ float strided_sum(const float* __restrict__ x, size_t stride, uint32_t n, float s) {
+    constexpr uint32_t U = 16;
+    uint32_t c = 0;
+    for (; c + U <= n; c += U) {
+        float v[U];
+#pragma unroll
+        for (uint32_t k = 0; k < U; k++) v[k] = x[(c + k) * stride];
+#pragma unroll
+        for (uint32_t k = 0; k < U; k++) s += v[k];
+    }
+    if (c < n) {
+        float v[U];
+#pragma unroll
+        for (uint32_t k = 0; k < U; k++) v[k] = x[(c + k < n ? c + k : c) * stride];
+#pragma unroll
+        for (uint32_t k = 0; k < U; k++)
+            if (c + k < n) s += v[k];
+    }
+    return s;
+}
 // Chunk partials summed within groups of GRAD_GROUP chunks, in place into
 // the group's first chunk row; grid (param blocks, groups).
 __global__ __launch_bounds__(256) void group_reduce_kernel(float* __restrict__ part, uint32_t chunks, uint32_t ptot) {
     const uint32_t p = blockIdx.x * 256 + threadIdx.x;
     const uint32_t c0 = blockIdx.y * GRAD_GROUP;
     if (p >= ptot || c0 >= chunks) return;
-    const uint32_t end = c0 + GRAD_GROUP < chunks ? c0 + GRAD_GROUP : chunks;
-    float s = 0.0f;
-    for (uint32_t c = c0; c < end; c++) s += part[size_t(c) * ptot + p];
-    part[size_t(c0) * ptot + p] = s;
+    const uint32_t n = chunks - c0 < GRAD_GROUP ? chunks - c0 : GRAD_GROUP;
+    float* x = part + size_t(c0) * ptot + p;
+    *x = strided_sum(x, ptot, n, 0.0f);
 }
-// Sequential sum over the group sums: grad[p] = 0 + g0[p] + g1[p] + ...
+// Sequential sum over the group sums: grad[p] = 0 + g0[p] + g1[p] + ...; with
+// one group, over its chunk partials directly: grad[p] = 0 + (0 + c0[p] + ...).
 __global__ __launch_bounds__(256) void chunk_reduce_kernel(const float* __restrict__ part, float* __restrict__ grad,
                                                            uint32_t chunks, uint32_t ptot) {
     const uint32_t p = blockIdx.x * 256 + threadIdx.x;
     if (p >= ptot) return;
-    float total = 0.0f;
-    for (uint32_t c = 0; c < chunks; c += GRAD_GROUP) total += part[size_t(c) * ptot + p];
-    grad[p] = total;
+    const float* x = part + p;
+    grad[p] = chunks <= GRAD_GROUP
+                  ? 0.0f + strided_sum(x, ptot, chunks, 0.0f)
+                  : strided_sum(x, size_t(GRAD_GROUP) * ptot, (chunks + GRAD_GROUP - 1) / GRAD_GROUP, 0.0f);
 }
 
-// ---------------------------------------------------------------- minibatches of one chunk
-// A minibatch of at most 256 rows is one gradient chunk, so every parameter's
-// sum runs over its rows in order (the reference's own order at its 256-row
-// minibatch).  chunk_kernel would run it in one workgroup; here the rows'
-// forward, objective and hidden deltas run in ceil(b/16) workgroups and the
-// parameter sums in 69 more, each chain still over the rows ascending:
+// ---------------------------------------------------------------- minibatches of few chunks
+// chunk_kernel runs a chunk of 256 rows in one workgroup, about 60 us of one
+// CU's time whatever the number of chunks, so minibatches of fewer chunks
+// than the GPU has CUs leave most of it idle.  Here the rows' forward,
+// objective and hidden deltas run in ceil(b/16) workgroups and the parameter
+// sums in 69 more per chunk, each chain still over the chunk's rows
+// ascending:
 //   mb_forward_kernel: 16 rows per workgroup, wavefronts 0-3 take the actor's
 //     hidden units 16w..16w+15 and 4-7 the critic's on 16x16x4 fp32 MFMA
 //     chains over the inputs from the bias (the fma chain of chunk_forward);
@@ -961,11 +985,11 @@ __global__ __launch_bounds__(256) void chunk_reduce_kernel(const float* __restri
 //     the hidden deltas, all written to the row records;
 //   mb_grad_kernel: every parameter's sum as a 16x16x4 MFMA chain over the
 //     rows, one 16x16 tile per wavefront (below).
-// Each gradient is stored as 0 + (0 + sum), the value the chunk reduction
-// (group sum from 0, then the sum of groups from 0) gives for one chunk.
+// A minibatch of one chunk (ONE) is the reference's own (256 rows): its
+// gradient needs no chunk reduction.
 constexpr uint32_t MB_HA = 0, MB_DA = 256 * 64, MB_HC = 2 * 256 * 64, MB_DC = 3 * 256 * 64, MB_RS = 4 * 256 * 64;
 constexpr uint32_t MB_FWD_ROWS = 16;
-template <uint32_t D>
+template <uint32_t D, bool ONE>
 __global__ __launch_bounds__(512) void mb_forward_kernel(MbArgs m) {
     using L = AL<D>;
     const RowArgs& a = m.r;
@@ -983,6 +1007,7 @@ __global__ __launch_bounds__(512) void mb_forward_kernel(MbArgs m) {
     const uint32_t t = threadIdx.x, wv = t / 64, l = t % 64;
     const uint32_t n0 = blockIdx.x * MB_FWD_ROWS;
     const uint32_t live_rows = a.b - n0 < MB_FWD_ROWS ? a.b - n0 : MB_FWD_ROWS;
+    float* rec = m.rec + (ONE ? 0 : size_t(n0 / CHUNK) * MB_REC_WORDS);  // this chunk's records
     constexpr uint32_t AT = 5 * HID + 8;  // actor tail words from b1 on
     float* s_at = s_t;
     float* s_ct = s_t + AT;
@@ -1106,7 +1131,7 @@ __global__ __launch_bounds__(512) void mb_forward_kernel(MbArgs m) {
     {   // hidden deltas (ppo.metal:470-485, 618-631) and the row records
         const uint32_t r = t / 32, k0 = t % 32;
         const bool live = r < live_rows;
-        const size_t row = n0 + r;
+        const size_t row = (ONE ? n0 : n0 % CHUNK) + r;
 #pragma unroll
         for (uint32_t u = 0; u < 2; u++) {
             const uint32_t k = k0 + 32 * u;
@@ -1114,12 +1139,12 @@ __global__ __launch_bounds__(512) void mb_forward_kernel(MbArgs m) {
 #pragma unroll
             for (uint32_t q = 0; q < 4; q++) d = fma_f(s_rs[r][q], w2[q * HID + k], d);
             const float ha = s_ha[r][k], hc = s_hc[r][k];
-            m.rec[MB_HA + row * HID + k] = ha;
-            m.rec[MB_DA + row * HID + k] = live ? d * (1.0f - ha * ha) : 0.0f;
-            m.rec[MB_HC + row * HID + k] = hc;
-            m.rec[MB_DC + row * HID + k] = live ? s_rs[r][12] * cw2[k] * (1.0f - hc * hc) : 0.0f;
+            rec[MB_HA + row * HID + k] = ha;
+            rec[MB_DA + row * HID + k] = live ? d * (1.0f - ha * ha) : 0.0f;
+            rec[MB_HC + row * HID + k] = hc;
+            rec[MB_DC + row * HID + k] = live ? s_rs[r][12] * cw2[k] * (1.0f - hc * hc) : 0.0f;
         }
-        if (k0 < 16) m.rec[MB_RS + row * 16 + k0] = s_rs[r][k0];
+        if (k0 < 16) rec[MB_RS + row * 16 + k0] = s_rs[r][k0];
     }
 }
 
@@ -1139,14 +1164,18 @@ template <uint32_t D>
 constexpr uint32_t mb_actor_in_tiles() { return (D + 1 + 15) / 16; }
 template <uint32_t D>
 constexpr uint32_t mb_tiles() { return 4 * mb_actor_in_tiles<D>() + 4 * ((COBS + 1 + 15) / 16) + 5 + 4; }
-template <uint32_t D>
+template <uint32_t D, bool ONE>
 __global__ __launch_bounds__(64) void mb_grad_kernel(MbArgs m) {
     using L = AL<D>;
     const RowArgs& a = m.r;
-    const uint32_t l = threadIdx.x, rows = a.b;
+    const uint32_t l = threadIdx.x, chunk = ONE ? 0 : blockIdx.y, n0 = chunk * CHUNK;
+    const uint32_t rows = ONE || a.b - n0 < CHUNK ? a.b - n0 : CHUNK;
+    const float* rec = m.rec + size_t(chunk) * MB_REC_WORDS;
+    const float* obs = a.obs + size_t(n0) * D;
+    const float* co = a.co + size_t(n0) * COBS;
     constexpr uint32_t AIT = mb_actor_in_tiles<D>(), CIT = (COBS + 1 + 15) / 16;
     constexpr uint32_t A_W1 = 4 * AIT, C_W1 = A_W1 + 4 * CIT, A_RS = C_W1 + 5;
-    const float* RS = m.rec + MB_RS;
+    const float* RS = rec + MB_RS;
     uint32_t tile = blockIdx.x;
     // operand sources: A[row][r] = arow(r), B[r][col] = bcol(r)
     uint32_t kind;  // 0 actor W1, 1 critic W1, 2 actor row scalars, 3 critic row scalars
@@ -1165,17 +1194,17 @@ __global__ __launch_bounds__(64) void mb_grad_kernel(MbArgs m) {
     uint32_t sa, sb;
     bool a_ok = true, b_ok, b_one;
     if (kind == 0) {
-        pa = m.rec + MB_DA + ar; sa = HID;
-        b_ok = bc < D; b_one = bc == D; pb = a.obs + (b_ok ? bc : 0); sb = D;
+        pa = rec + MB_DA + ar; sa = HID;
+        b_ok = bc < D; b_one = bc == D; pb = obs + (b_ok ? bc : 0); sb = D;
     } else if (kind == 1) {
-        pa = m.rec + MB_DC + ar; sa = HID;
-        b_ok = bc < COBS; b_one = bc == COBS; pb = a.co + (b_ok ? bc : 0); sb = COBS;
+        pa = rec + MB_DC + ar; sa = HID;
+        b_ok = bc < COBS; b_one = bc == COBS; pb = co + (b_ok ? bc : 0); sb = COBS;
     } else if (kind == 2) {
         a_ok = ar < 13; pa = RS + (a_ok ? ar : 0); sa = 16;
-        b_ok = bc < HID; b_one = bc == HID; pb = m.rec + MB_HA + (b_ok ? bc : 0); sb = HID;
+        b_ok = bc < HID; b_one = bc == HID; pb = rec + MB_HA + (b_ok ? bc : 0); sb = HID;
     } else {
         a_ok = ar < 13; pa = RS + (a_ok ? ar : 0); sa = 16;
-        b_ok = true; b_one = false; pb = m.rec + MB_HC + bc; sb = HID;
+        b_ok = true; b_one = false; pb = rec + MB_HC + bc; sb = HID;
     }
     const float b_pad = b_one ? 1.0f : -0.0f;
     float xv[64], yv[64];
@@ -1198,13 +1227,15 @@ __global__ __launch_bounds__(64) void mb_grad_kernel(MbArgs m) {
         const float bv = rv ? (b_ok ? yv[s] : b_pad) : -0.0f;
         acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, acc, 0, 0, 0);
     }
-    float* g = m.grad;
+    // a single chunk's sums are the gradient (0 + (0 + sum), as the chunk
+    // reduction would form it); several leave partials for that reduction
+    float* g = ONE ? m.grad : a.part + size_t(chunk) * L::P_TOTAL;
     // accumulator register r of lane l holds D[4 (l/16) + r][l % 16]
 #pragma unroll
     for (uint32_t r = 0; r < 4; r++) {
         const uint32_t row = 16 * jt + 4 * (l / 16) + r;  // A row of this value
         const uint32_t col = bc;
-        const float val = 0.0f + (0.0f + acc[r]);
+        const float val = ONE ? 0.0f + (0.0f + acc[r]) : acc[r];
         int32_t out = -1;
         if (kind == 0) {
             if (col < D) out = int32_t(row * D + col);
@@ -1352,6 +1383,13 @@ __global__ void metric_mean_kernel(const float* __restrict__ rows, float* __rest
     for (int k = 0; k < 4; k++) mean[k] = updates ? s[k] / float(updates) : 0.0f;
 }
 
+template <uint32_t D, bool ONE>
+void launch_minibatch(const MbArgs& m, uint32_t chunks, hipStream_t st) {
+    const dim3 fwd((m.r.b + MB_FWD_ROWS - 1) / MB_FWD_ROWS);
+    hipLaunchKernelGGL((mb_forward_kernel<D, ONE>), fwd, dim3(512), 0, st, m);
+    hipLaunchKernelGGL((mb_grad_kernel<D, ONE>), dim3(mb_tiles<D>(), chunks), dim3(64), 0, st, m);
+}
+
 }  // namespace ppo
 
 // ---------------------------------------------------------------- launchers
@@ -1422,23 +1460,15 @@ hipError_t ppo_launch_rows(const ppo::RowArgs* a, hipStream_t st) {
     return hipGetLastError();
 }
 
-// A minibatch of at most 256 rows: forward/objective/deltas, then the
-// finished gradient in grad (no chunk reduction).
+// A minibatch of at most MB_MAX_CHUNKS chunks: forward/objective/deltas, then
+// the finished gradient in grad (one chunk) or the chunks' partials in part
+// (ppo_launch_grads reduces them).
 hipError_t ppo_launch_minibatch(const ppo::MbArgs* m, hipStream_t st) {
-    const uint32_t b = m->r.b;
-    if (b == 0 || b > ppo::MB_ROWS) return hipErrorInvalidValue;
-    const dim3 fwd((b + ppo::MB_FWD_ROWS - 1) / ppo::MB_FWD_ROWS);
-    if (m->r.d == MDN_ACTOR_OBS_POOLED) {
-        hipLaunchKernelGGL(ppo::mb_forward_kernel<MDN_ACTOR_OBS_POOLED>, fwd, dim3(512), 0, st, *m);
-        hipLaunchKernelGGL(ppo::mb_grad_kernel<MDN_ACTOR_OBS_POOLED>,
-                           dim3(ppo::mb_tiles<MDN_ACTOR_OBS_POOLED>()), dim3(64), 0, st, *m);
-    } else if (m->r.d == MDN_ACTOR_OBS_PRIOR) {
-        hipLaunchKernelGGL(ppo::mb_forward_kernel<MDN_ACTOR_OBS_PRIOR>, fwd, dim3(512), 0, st, *m);
-        hipLaunchKernelGGL(ppo::mb_grad_kernel<MDN_ACTOR_OBS_PRIOR>,
-                           dim3(ppo::mb_tiles<MDN_ACTOR_OBS_PRIOR>()), dim3(64), 0, st, *m);
-    } else {
-        return hipErrorInvalidValue;
-    }
+    constexpr uint32_t P = MDN_ACTOR_OBS_POOLED, H = MDN_ACTOR_OBS_PRIOR;
+    const uint32_t chunks = (m->r.b + ppo::CHUNK - 1) / ppo::CHUNK;
+    if (chunks == 0 || chunks > ppo::MB_MAX_CHUNKS || (m->r.d != P && m->r.d != H)) return hipErrorInvalidValue;
+    if (m->r.d == P) chunks == 1 ? ppo::launch_minibatch<P, true>(*m, 1, st) : ppo::launch_minibatch<P, false>(*m, chunks, st);
+    else chunks == 1 ? ppo::launch_minibatch<H, true>(*m, 1, st) : ppo::launch_minibatch<H, false>(*m, chunks, st);
     return hipGetLastError();
 }
 
@@ -1446,7 +1476,9 @@ hipError_t ppo_launch_grads(float* part, float* grad, uint32_t b, uint32_t d, hi
     const uint32_t chunks = (b + ppo::CHUNK - 1) / ppo::CHUNK;
     const uint32_t groups = (chunks + ppo::GRAD_GROUP - 1) / ppo::GRAD_GROUP;
     const uint32_t ptot = ppo_partial_stride(d);
-    hipLaunchKernelGGL(ppo::group_reduce_kernel, dim3((ptot + 255) / 256, groups), dim3(256), 0, st, part, chunks, ptot);
+    if (groups > 1)
+        hipLaunchKernelGGL(ppo::group_reduce_kernel, dim3((ptot + 255) / 256, groups), dim3(256), 0, st, part, chunks,
+                           ptot);
     hipLaunchKernelGGL(ppo::chunk_reduce_kernel, dim3((ptot + 255) / 256), dim3(256), 0, st, part, grad, chunks, ptot);
     return hipGetLastError();
 }

@@ -1,9 +1,10 @@
 """The sizes at which a kernel or its split of the work changes, against the
 oracle at tolerance 0: fleets around the small-fleet rollout's envs per
 wavefront (1,024 envs each) and its limit (4,096), with every ring size, the
-guided actor and per-episode plants."""
+guided actor and per-episode plants; minibatches around the few-chunk limit."""
 import sys
 
+import numpy as np
 import pytest
 
 from gpu_compare import ENV_BUFFERS, ROW_BUFFERS, compare, config, make_pair
@@ -60,3 +61,38 @@ def test_fleet_plants_and_tasks(n, delay, obs):
         x.set_runtime(rt)
         x.set_tasks(t)
     _collect_both(sim, ora, 6, ["environment_physics", "task_states"])
+
+
+@pytest.mark.parametrize("obs", [181, 184])
+@pytest.mark.parametrize("n,T,minibatch", [(257, 1, 257), (64, 8, 512), (100, 83, 4150), (2048, 10, 20480),
+                                           (20481, 1, 20481)])
+def test_few_chunk_minibatches(obs, n, T, minibatch):
+    """One chunk more than the single-chunk path, two chunks, an odd last
+    chunk in two minibatches, the most chunks of the few-chunk path and one
+    more (the chunk kernel); the update is the oracle's bit for bit."""
+    say("case: update of %d x %d rows, minibatches of %d, %d inputs" % (n, T, minibatch, obs))
+    sim, ppo, ora = make_pair(config(n=n, family=1, seed=3, max_steps=7), T, epochs=2, minibatch=minibatch,
+                              actor_obs=obs)
+    rng = np.random.default_rng(n)
+    for name in ("actor", "critic"):
+        w = sim.get(name)
+        w *= (1.0 + 0.1 * rng.standard_normal(w.size)).astype(np.float32)
+        sim.set(name, w)
+        ora.set(name, w)
+    sim.collect()
+    ora.collect()
+    for it in range(2):
+        ppo.rollout_update(it)
+        ora.gae()
+        ora.normalize()
+        ora.update(it)
+    names = ["actor", "critic", "actor_m", "actor_v", "critic_m", "critic_v", "advantages", "returns", "metric_rows",
+             "grad_norm_rows"]
+    bad = compare(sim, ora, names)
+    assert not bad, bad
+    assert np.array_equal(ppo.metric_mean(), ora.metric_mean())
+    # the rollout's transposed first layers follow the update
+    sim.collect()
+    ora.collect()
+    bad = compare(sim, ora, ENV_BUFFERS + ROW_BUFFERS)
+    assert not bad, bad
