@@ -247,10 +247,25 @@ __global__ __launch_bounds__(256) void gae_kernel(const float* __restrict__ r, c
 constexpr uint32_t NORM_THREADS = 1024, NORM_WAVE_CHUNKS = NORM_GROUP / (NORM_THREADS / 64);
 static_assert(NORM_WAVE_CHUNKS * (NORM_THREADS / 64) == NORM_GROUP, "a workgroup per group of chunks");
 
+// v of the lane that DPP control CTRL names (every lane has a source).
+template <int CTRL>
+__device__ __forceinline__ double dpp_double(double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const int lo = __builtin_amdgcn_update_dpp(0, int(uint32_t(b)), CTRL, 0xF, 0xF, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, int(uint32_t(b >> 32)), CTRL, 0xF, 0xF, false);
+    return __builtin_bit_cast(double, (uint64_t(uint32_t(hi)) << 32) | uint32_t(lo));
+}
 // Sum of the 64 lanes' values in the canonical tree (xor levels 1..32).
+// Levels 1 and 2 swap within quads; after them the lanes of a quad are equal,
+// so mirroring a half row is level 4, and mirroring a row level 8; the two
+// levels across rows shuffle through LDS.
 __device__ __forceinline__ double chunk_tree(double v) {
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) v = v + __shfl_xor(v, off, 64);
+    v = v + dpp_double<0xB1>(v);   // quad_perm [1,0,3,2]
+    v = v + dpp_double<0x4E>(v);   // quad_perm [2,3,0,1]
+    v = v + dpp_double<0x141>(v);  // row_half_mirror
+    v = v + dpp_double<0x140>(v);  // row_mirror
+    v = v + __shfl_xor(v, 16, 64);
+    v = v + __shfl_xor(v, 32, 64);
     return v;
 }
 // Sequential sum of p[0, m) (the group partials, in order), returned to
@@ -379,6 +394,100 @@ __global__ __launch_bounds__(NORM_THREADS) void norm_pass_kernel(const float* __
     if (!s_last) return;
     const double total = sequential_total(p1, groups, threadIdx.x < groups ? p1[threadIdx.x] : 0.0, sp);
     if (threadIdx.x == 0) stats[1] = 1.0f / sqrt_f(float(total / double(count)) + eps);
+}
+// At most NORM_SMALL_GROUPS groups: both passes and the rescale in one
+// workgroup that holds the values in registers (16 per thread and group; four
+// groups' do not fit).  The three launches of the general path are launch
+// ramps and dependent round trips at these sizes (4,096 values: 15.5 us),
+// which one launch takes once (6.9 us).  Same partials in the same order:
+// chunk trees, the chunks of a group in order (one thread per group), then
+// the groups.
+constexpr uint32_t NORM_SMALL_GROUPS = 2;
+template <bool A16, uint32_t NG>
+__global__ __launch_bounds__(NORM_THREADS) void norm_small_kernel(float* __restrict__ a, uint32_t count,
+                                                                  float* __restrict__ stats, float eps, int apply) {
+    __shared__ double s_chunk[NG][NORM_GROUP];
+    __shared__ double s_group[NG];
+    const uint32_t chunks = (count + CHUNK - 1) / CHUNK, groups = (chunks + NORM_GROUP - 1) / NORM_GROUP;
+    const uint32_t w = threadIdx.x / 64, l = threadIdx.x % 64;
+    float x[NG][NORM_WAVE_CHUNKS][4];
+#pragma unroll
+    for (uint32_t g = 0; g < NG; g++)
+#pragma unroll
+        for (uint32_t i = 0; i < NORM_WAVE_CHUNKS; i++) {
+            const uint32_t e = (g * NORM_GROUP + NORM_WAVE_CHUNKS * w + i) * CHUNK + 4 * l;
+            if (A16 && e + 3 < count) {
+                const float4 v4 = *reinterpret_cast<const float4*>(a + e);
+                x[g][i][0] = v4.x; x[g][i][1] = v4.y; x[g][i][2] = v4.z; x[g][i][3] = v4.w;
+            } else {
+#pragma unroll
+                for (uint32_t j = 0; j < 4; j++) x[g][i][j] = e + j < count ? a[e + j] : 0.0f;
+            }
+        }
+    float mean = 0.0f, inv = 0.0f;
+#pragma unroll
+    for (int pass = 0; pass < 2; pass++) {
+#pragma unroll
+        for (uint32_t g = 0; g < NG; g++) {
+            // one group's trees at a time: their temporaries fit beside the values
+            if (g) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (uint32_t i = 0; i < NORM_WAVE_CHUNKS; i++) {
+                const uint32_t c = NORM_WAVE_CHUNKS * w + i, e = (g * NORM_GROUP + c) * CHUNK + 4 * l;
+                double s = 0.0;
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j)
+                    if (e + j < count) {
+                        const double d = pass == 0 ? double(x[g][i][j]) : double(x[g][i][j] - mean);
+                        s += pass == 0 ? d : d * d;
+                    }
+                s = chunk_tree(s);
+                if (l == 0) s_chunk[g][c] = s;
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x < groups) {
+            const uint32_t g = threadIdx.x;
+            const uint32_t k = chunks - g * NORM_GROUP < NORM_GROUP ? chunks - g * NORM_GROUP : NORM_GROUP;
+            double v = 0.0;
+#pragma unroll
+            for (uint32_t c = 0; c < NORM_GROUP; c += 16) {
+                double y[16];
+#pragma unroll
+                for (uint32_t j = 0; j < 16; j++) y[j] = s_chunk[g][c + j];
+#pragma unroll
+                for (uint32_t j = 0; j < 16; j++)
+                    if (c + j < k) v += y[j];
+            }
+            s_group[g] = v;
+        }
+        __syncthreads();
+        double total = 0.0;
+#pragma unroll
+        for (uint32_t g = 0; g < NG; g++)
+            if (g < groups) total += s_group[g];
+        if (pass == 0) mean = float(total / double(count));
+        else inv = 1.0f / sqrt_f(float(total / double(count)) + eps);
+    }
+    if (threadIdx.x == 0) {
+        stats[0] = mean;
+        stats[1] = inv;
+    }
+    if (!apply) return;
+#pragma unroll
+    for (uint32_t g = 0; g < NG; g++)
+#pragma unroll
+        for (uint32_t i = 0; i < NORM_WAVE_CHUNKS; i++) {
+            const uint32_t e = (g * NORM_GROUP + NORM_WAVE_CHUNKS * w + i) * CHUNK + 4 * l;
+            if (A16 && e + 3 < count) {
+                *reinterpret_cast<float4*>(a + e) = make_float4((x[g][i][0] - mean) * inv, (x[g][i][1] - mean) * inv,
+                                                                (x[g][i][2] - mean) * inv, (x[g][i][3] - mean) * inv);
+            } else {
+#pragma unroll
+                for (uint32_t j = 0; j < 4; j++)
+                    if (e + j < count) a[e + j] = (x[g][i][j] - mean) * inv;
+            }
+        }
 }
 // (a - mean) * inv over the workgroup's NORM_APPLY elements (loaded at
 // once), with (mean, inv) from stats.
@@ -1374,13 +1483,37 @@ __global__ __launch_bounds__(256) void transpose_w1_kernel(const float* __restri
     }
 }
 
-// metric_mean (main.mm:952-962): sequential over updates.
-__global__ void metric_mean_kernel(const float* __restrict__ rows, float* __restrict__ mean, uint32_t updates) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    float s[4] = {0, 0, 0, 0};
-    for (uint32_t u = 0; u < updates; u++)
-        for (int k = 0; k < 4; k++) s[k] += rows[size_t(u) * 4 + k];
-    for (int k = 0; k < 4; k++) mean[k] = updates ? s[k] / float(updates) : 0.0f;
+// metric_mean (main.mm:952-962): sequential over updates.  Rounds of 256
+// rows go through LDS (one coalesced load per round and thread); lane q < 4
+// adds metric q's rows in order, the next round's load in flight beneath the
+// adds (one thread adding straight from memory took 185 us for 2,048 rows,
+// this 14 us).
+__global__ __launch_bounds__(256) void metric_mean_kernel(const float4* __restrict__ rows, float* __restrict__ mean,
+                                                          uint32_t updates) {
+    __shared__ float s_row[4][256 + 1];
+    const uint32_t t = threadIdx.x;
+    const float4 zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float4 next = t < updates ? rows[t] : zero;
+    float s = 0.0f;
+    for (uint32_t u0 = 0; u0 < updates; u0 += 256) {
+        s_row[0][t] = next.x; s_row[1][t] = next.y; s_row[2][t] = next.z; s_row[3][t] = next.w;
+        __syncthreads();
+        if (u0 + 256 < updates) next = u0 + 256 + t < updates ? rows[u0 + 256 + t] : zero;
+        if (t < 4) {
+            const uint32_t k = updates - u0 < 256 ? updates - u0 : 256;
+            uint32_t u = 0;
+            for (; u + 16 <= k; u += 16) {
+                float v[16];
+#pragma unroll
+                for (uint32_t j = 0; j < 16; j++) v[j] = s_row[t][u + j];
+#pragma unroll
+                for (uint32_t j = 0; j < 16; j++) s += v[j];
+            }
+            for (; u < k; u++) s += s_row[t][u];
+        }
+        __syncthreads();
+    }
+    if (t < 4) mean[t] = updates ? s / float(updates) : 0.0f;
 }
 
 template <uint32_t D, bool ONE>
@@ -1430,6 +1563,13 @@ hipError_t ppo_launch_normalize_stats(float* a, uint64_t count, double* part, fl
     const uint64_t applies = (count + ppo::NORM_APPLY - 1) / ppo::NORM_APPLY;
     if (groups > 0x7fffffffull || applies > 0x7fffffffull) return hipErrorInvalidValue;
     const bool a16 = reinterpret_cast<uintptr_t>(a) % 16 == 0;
+    if (groups <= ppo::NORM_SMALL_GROUPS) {
+        auto* kernel = groups == 1 ? (a16 ? ppo::norm_small_kernel<true, 1> : ppo::norm_small_kernel<false, 1>)
+                                   : (a16 ? ppo::norm_small_kernel<true, ppo::NORM_SMALL_GROUPS>
+                                          : ppo::norm_small_kernel<false, ppo::NORM_SMALL_GROUPS>);
+        hipLaunchKernelGGL(kernel, dim3(1), dim3(ppo::NORM_THREADS), 0, st, a, uint32_t(count), stats, eps, apply);
+        return hipGetLastError();
+    }
     for (int pass = 0; pass < 2; pass++) {
         if (a16)
             hipLaunchKernelGGL(ppo::norm_pass_kernel<true>, dim3(uint32_t(groups)), dim3(ppo::NORM_THREADS), 0, st, a,
@@ -1509,7 +1649,8 @@ hipError_t ppo_launch_transpose(const float* actor, const float* critic, float* 
 }
 
 hipError_t ppo_launch_metric_mean(const float* rows, float* mean, uint32_t updates, hipStream_t st) {
-    hipLaunchKernelGGL(ppo::metric_mean_kernel, dim3(1), dim3(64), 0, st, rows, mean, updates);
+    hipLaunchKernelGGL(ppo::metric_mean_kernel, dim3(1), dim3(256), 0, st, reinterpret_cast<const float4*>(rows), mean,
+                       updates);
     return hipGetLastError();
 }
 

@@ -1,14 +1,17 @@
 """The sizes at which a kernel or its split of the work changes, against the
 oracle at tolerance 0: fleets around the small-fleet rollout's envs per
 wavefront (1,024 envs each) and its limit (4,096), with every ring size, the
-guided actor and per-episode plants; minibatches around the few-chunk limit."""
+guided actor and per-episode plants; minibatches around the few-chunk limit;
+advantage normalisation around a chunk, a group and the one-workgroup limit."""
+import ctypes
 import sys
 
 import numpy as np
 import pytest
 
 from gpu_compare import ENV_BUFFERS, ROW_BUFFERS, compare, config, make_pair
-from mdnav import task_runtime, task_settings
+from mdnav import native, ops, task_runtime, task_settings
+from oracle_lib import oracle, ptr
 
 pytestmark = pytest.mark.gpu
 
@@ -96,3 +99,40 @@ def test_few_chunk_minibatches(obs, n, T, minibatch):
     ora.collect()
     bad = compare(sim, ora, ENV_BUFFERS + ROW_BUFFERS)
     assert not bad, bad
+
+
+@pytest.mark.parametrize("updates", [1, 15, 256, 257, 530])
+def test_metric_mean_rows(updates):
+    say("case: metric mean over", updates, "updates")
+    sim, ppo, ora = make_pair(config(n=updates, family=1, seed=3), 3, epochs=1, minibatch=3)
+    sim.collect()
+    ppo.rollout_update(0)
+    rows = sim.get("metric_rows").reshape(updates, 4)
+    want = np.zeros(4, np.float32)
+    for r in rows:
+        want = want + r
+    assert np.array_equal(ppo.metric_mean(), want / np.float32(updates))
+
+
+@pytest.mark.parametrize("count", [1, 2, 255, 256, 257, 4097, 16383, 16384, 16385, 32767, 32768, 32769, 65537])
+def test_normalize_sizes(count):
+    from test_zz_no_alloc import hip_runtime
+    say("case: normalise", count, "values")
+    rng = np.random.default_rng(count)
+    x = rng.normal(3, 5, count).astype(np.float32)
+    want = x.copy()
+    oracle().orc_normalize_advantages(ptr(want), count, np.float32(1e-8))
+    assert np.array_equal(ops.normalize(x), want)
+    # device memory at every 4-byte alignment, with values before and after left alone
+    hip = hip_runtime()
+    for offset in (0, 1, 2, 3):
+        host = np.full(count + 8, 7.0, np.float32)
+        host[offset:offset + count] = x
+        dev = ctypes.c_void_p()
+        assert hip.hipMalloc(ctypes.byref(dev), host.nbytes) == 0
+        assert hip.hipMemcpy(dev, ptr(host), host.nbytes, 1) == 0
+        native.check(native.lib().mdn_op_normalize_noalloc(ctypes.c_void_p(dev.value + 4 * offset), count, 1e-8, None))
+        assert hip.hipMemcpy(ptr(host), dev, host.nbytes, 2) == 0
+        assert hip.hipFree(dev) == 0
+        assert np.array_equal(host[offset:offset + count], want), offset
+        assert np.all(host[:offset] == 7.0) and np.all(host[offset + count:] == 7.0)
