@@ -2,7 +2,8 @@
 oracle at tolerance 0: fleets around the small-fleet rollout's envs per
 wavefront (1,024 envs each) and its limit (4,096), with every ring size, the
 guided actor and per-episode plants; minibatches around the few-chunk limit;
-advantage normalisation around a chunk, a group and the one-workgroup limit."""
+advantage normalisation around a chunk, a group and the one-workgroup limit;
+the geometry memory either side of its wide workgroups."""
 import ctypes
 import sys
 
@@ -64,6 +65,14 @@ def test_fleet_plants_and_tasks(n, delay, obs):
         x.set_runtime(rt)
         x.set_tasks(t)
     _collect_both(sim, ora, 6, ["environment_physics", "task_states"])
+
+
+@pytest.mark.parametrize("n", [2048, 2049])
+def test_memory_workgroups(n):
+    say("case: geometry memory, fleet of", n)
+    cfg = config(n=n, family=12, seed=11, speed=1.5, distance=4.0, geometry_memory=1)
+    sim, _, ora = make_pair(cfg, 9, actor_obs=184)
+    _collect_both(sim, ora, 9)
 
 
 @pytest.mark.parametrize("obs", [181, 184])
