@@ -194,7 +194,10 @@ typedef float v4f __attribute__((ext_vector_type(4)));
 // The operands of k-step s are read from LDS PF steps before its MFMAs issue
 // (a scheduling fence between steps keeps that order), so the LDS latency of
 // one step overlaps the matrix-core work of the previous ones.
-constexpr uint32_t MFMA_PF = 3;
+// A small fleet's wavefront has one tile per step instead of two and reads
+// twice as far ahead.
+template <bool S>
+constexpr uint32_t mfma_pf() { return S ? 6 : 3; }
 // How the four wavefronts cover the workgroup's envs (LDS rows):
 //   32 envs (8 per wavefront): wavefront w takes tiles 2w and 2w + 1 of the
 //     2 x 4 grid of 16x16 tiles (env block w/2, one A operand for both);
@@ -212,8 +215,30 @@ struct TileMap {
 #pragma unroll
         for (uint32_t q = 0; q < NT; q++) unit[q] = S ? 16 * wv + l % 16 : 16 * ((2 * wv + q) % 4) + l % 16;
     }
-    __device__ __forceinline__ bool stored(uint32_t r) const { return !S || e0 + r < envs; }
 };
+// tanh of a small fleet's accumulators into out[env][unit].  With 4 or 8 envs
+// per workgroup the tile's rows repeat, so each quarter of the lanes evaluates
+// its share of the envs: one or two values per lane, not four.
+template <uint32_t OS>
+__device__ __forceinline__ void store_small(const TileMap<true>& tm, const v4f& acc, float* out) {
+    const uint32_t kq = threadIdx.x % 64 / 16, unit = tm.unit[0];
+    const float a0 = acc[0], a1 = acc[1], a2 = acc[2], a3 = acc[3];
+    if (tm.envs == 4) {
+        out[kq * OS + unit] = tanh_f(kq == 0 ? a0 : kq == 1 ? a1 : kq == 2 ? a2 : a3);
+    } else if (tm.envs == 8) {
+        const bool lo = kq < 2;
+        const uint32_t row = 4 * (kq % 2) + (lo ? 0 : 2);
+        const float v0 = lo ? a0 : a2, v1 = lo ? a1 : a3;
+        out[row * OS + unit] = tanh_f(v0);
+        out[(row + 1) * OS + unit] = tanh_f(v1);
+    } else {
+#pragma unroll
+        for (uint32_t r = 0; r < 4; r++) {
+            const float h = tanh_f(acc[r]);
+            if (tm.e0 + r < tm.envs) out[(tm.e0 + r) * OS + unit] = h;
+        }
+    }
+}
 template <uint32_t D, uint32_t XS, uint32_t OS, bool S>
 __device__ __forceinline__ void wg_layer(uint32_t envs, const float* x, const float* w1t, const float* b1,
                                          float* out) {
@@ -226,7 +251,7 @@ __device__ __forceinline__ void wg_layer(uint32_t envs, const float* x, const fl
         const float bias = b1[tm.unit[q]];
         acc[q][0] = bias; acc[q][1] = bias; acc[q][2] = bias; acc[q][3] = bias;
     }
-    constexpr uint32_t NK = (D + 3) / 4;
+    constexpr uint32_t NK = (D + 3) / 4, MFMA_PF = mfma_pf<S>();
     float av[NK], bv[NK][NT];
 #pragma unroll
     for (uint32_t st = 0; st < NK + MFMA_PF; st++) {
@@ -243,13 +268,14 @@ __device__ __forceinline__ void wg_layer(uint32_t envs, const float* x, const fl
         }
         __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (S) {
+        store_small<OS>(tm, acc[0], out);
+    } else {
 #pragma unroll
-    for (uint32_t q = 0; q < NT; q++)
+        for (uint32_t q = 0; q < NT; q++)
 #pragma unroll
-        for (uint32_t r = 0; r < 4; r++) {
-            const float h = tanh_f(acc[q][r]);
-            if (tm.stored(r)) out[(tm.e0 + r) * OS + tm.unit[q]] = h;
-        }
+            for (uint32_t r = 0; r < 4; r++) out[(tm.e0 + r) * OS + tm.unit[q]] = tanh_f(acc[q][r]);
+    }
 }
 
 // wg_layer with the weight operands already in registers: bw[q][kk] is
@@ -267,7 +293,7 @@ __device__ __forceinline__ void wg_layer_rb(uint32_t envs, const float* x,
         const float bias = b1[tm.unit[q]];
         acc[q][0] = bias; acc[q][1] = bias; acc[q][2] = bias; acc[q][3] = bias;
     }
-    constexpr uint32_t NK = D / 4;
+    constexpr uint32_t NK = D / 4, MFMA_PF = mfma_pf<S>();
     float av[NK];
 #pragma unroll
     for (uint32_t st = 0; st < NK + MFMA_PF; st++) {
@@ -279,13 +305,14 @@ __device__ __forceinline__ void wg_layer_rb(uint32_t envs, const float* x,
         }
         __builtin_amdgcn_sched_barrier(0);
     }
+    if constexpr (S) {
+        store_small<OS>(tm, acc[0], out);
+    } else {
 #pragma unroll
-    for (uint32_t q = 0; q < NT; q++)
+        for (uint32_t q = 0; q < NT; q++)
 #pragma unroll
-        for (uint32_t r = 0; r < 4; r++) {
-            const float h = tanh_f(acc[q][r]);
-            if (tm.stored(r)) out[(tm.e0 + r) * OS + tm.unit[q]] = h;
-        }
+            for (uint32_t r = 0; r < 4; r++) out[(tm.e0 + r) * OS + tm.unit[q]] = tanh_f(acc[q][r]);
+    }
 }
 // This lane's weight operands of wg_layer_rb for w1t[D][HID].
 template <uint32_t D, bool S>
@@ -314,7 +341,7 @@ __device__ __forceinline__ void wg_head(uint32_t envs, const float* x, const flo
     v4f acc;
     const float bias = c < NC ? b[c] : 0.0f;
     acc[0] = bias; acc[1] = bias; acc[2] = bias; acc[3] = bias;
-    constexpr uint32_t NK = HID / 4;
+    constexpr uint32_t NK = HID / 4, MFMA_PF = mfma_pf<S>();
     float av[NK], bv[NK];
 #pragma unroll
     for (uint32_t st = 0; st < NK + MFMA_PF; st++) {
@@ -377,8 +404,8 @@ __device__ __forceinline__ void raptor_operands(const float* RW, RaptorRegs& o) 
 // (stride 17).  Call from uniform control flow; `on` masks envs whose step
 // is skipped.
 // Small fleets (S): the wavefront holds epw <= 4 envs; tile row i is its env
-// i % epw, so quarter kq of the lanes takes rows 0, 1 (kq even) or 2, 3 (kq
-// odd) of its four and the quarters cover the envs between them.
+// i % epw, so among the four rows of each quarter kq of the lanes there is one
+// of env kq % epw: each lane evaluates the gates of one (env, unit) pair.
 template <int G, uint32_t MS, bool S>
 __device__ __forceinline__ void raptor_wave(const float* RW, const RaptorRegs& o, const float (&mo)[22], float* smo,
                                             float* sx, float* srh, uint32_t grp, uint32_t epw, bool on,
@@ -410,7 +437,7 @@ __device__ __forceinline__ void raptor_wave(const float* RW, const RaptorRegs& o
     // GRU gate products (raptor.hpp:62-84): gate g of unit u is row 16g + u.
     // Lane (kq, j) holds envs 4 kq + r (mod 8) of unit j; lanes kq < 2 keep
     // rows r = 0, 1 and lanes kq >= 2 rows 2, 3, so each env is taken once.
-    const bool lo = S ? kq % 2 == 0 : kq < 2;
+    const bool lo = kq < 2;
     float ax[4], ah[4];
 #pragma unroll
     for (uint32_t kk = 0; kk < 4; kk++) {
@@ -419,11 +446,14 @@ __device__ __forceinline__ void raptor_wave(const float* RW, const RaptorRegs& o
     }
     // one gate at a time (two chains live), each folded into the gate
     // values as soon as it is complete
-    float reset[2], update[2], nh[2], hold[2];
-    uint32_t e2[2];
+    constexpr uint32_t NP = S ? 1 : 2;  // gate values per lane
+    float reset[NP], update[NP], nh[NP], hold[NP];
+    uint32_t e2[NP];
+    // small fleets: the row of env kq % epw in quarter kq (4 kq + rsel = kq mod epw)
+    const uint32_t rsel = epw == 4 ? kq : epw == 2 ? kq % 2 : 0;
 #pragma unroll
-    for (uint32_t p = 0; p < 2; p++) {
-        e2[p] = base + (4 * kq + (lo ? p : 2 + p)) % (S ? epw : 8);
+    for (uint32_t p = 0; p < NP; p++) {
+        e2[p] = S ? base + kq % epw : base + (4 * kq + (lo ? p : 2 + p)) % 8;
         hold[p] = srh[e2[p] * 17 + j];
     }
 #pragma unroll
@@ -438,13 +468,22 @@ __device__ __forceinline__ void raptor_wave(const float* RW, const RaptorRegs& o
             ch = __builtin_amdgcn_mfma_f32_16x16x4f32(ah[kk], o.gh[g][kk], ch, 0, 0, 0);
         }
 #pragma unroll
-        for (uint32_t p = 0; p < 2; p++) {
+        for (uint32_t p = 0; p < NP; p++) {
             // rows p and 2 + p as two fixed registers and one select each (an
             // empty asm keeps the compiler from turning the pair into a
             // lane-dependent row index, which it expands to a compare chain)
             float i0 = ci[p], i2 = ci[2 + p], h0 = ch[p], h2 = ch[2 + p];
+            bool low = lo;
+            if constexpr (S) {
+                float i1 = ci[1], i3 = ci[3], h1 = ch[1], h3 = ch[3];
+                asm volatile("" : "+v"(i0), "+v"(i1), "+v"(h0), "+v"(h1));
+                asm volatile("" : "+v"(i2), "+v"(i3), "+v"(h2), "+v"(h3));
+                const bool odd = rsel & 1u;
+                i0 = odd ? i1 : i0; i2 = odd ? i3 : i2; h0 = odd ? h1 : h0; h2 = odd ? h3 : h2;
+                low = rsel < 2;
+            }
             asm volatile("" : "+v"(i0), "+v"(i2), "+v"(h0), "+v"(h2));
-            const float iv = lo ? i0 : i2, hv = lo ? h0 : h2;
+            const float iv = low ? i0 : i2, hv = low ? h0 : h2;
             if (g == 0) {
                 reset[p] = sigmoid_f(iv + hv);
             } else if (g == 1) {
@@ -456,12 +495,12 @@ __device__ __forceinline__ void raptor_wave(const float* RW, const RaptorRegs& o
         }
     }
     const uint64_t live = __ballot(on);
-    bool on2[2];
+    bool on2[NP];
 #pragma unroll
-    for (uint32_t p = 0; p < 2; p++) on2[p] = (live >> ((e2[p] - base) * G)) & 1ull;
+    for (uint32_t p = 0; p < NP; p++) on2[p] = (live >> ((e2[p] - base) * G)) & 1ull;
     group_sync();  // every lane's reads of the old hidden state precede the writes
 #pragma unroll
-    for (uint32_t p = 0; p < 2; p++)
+    for (uint32_t p = 0; p < NP; p++)
         if (on2[p]) srh[e2[p] * 17 + j] = nh[p];
     group_sync();
     {   // output dense + clip (raptor.hpp:86-97)
@@ -480,6 +519,31 @@ __device__ __forceinline__ void raptor_wave(const float* RW, const RaptorRegs& o
 }
 
 // ---------------------------------------------------------------- rollout
+// Words of MdnPhysicsParams that the standard quadrotor structure
+// (mdn::quad_structure) fixes, one bit per word: +0 (rotor heights, thrust and
+// torque directions off z, off-diagonal inertia and inverse, gravity off z),
+// 1 (thrust along z), 1 or -1 (torque about z).
+constexpr uint32_t quad_bits(uint32_t word, int what) {
+    uint32_t m = 0;
+    for (uint32_t i = 32 * word; i < 32 * word + 32; i++) {
+        const bool axis = i % 3 == 2;
+        const int kind = i < 12 ? (axis ? 0 : -1)
+                       : i < 24 ? (axis ? 1 : 0)
+                       : i < 36 ? (axis ? 2 : 0)
+                       : i >= 60 && i < 78 ? ((i - 60) % 9 % 4 ? 0 : -1)
+                       : i == 78 || i == 79 ? 0 : -1;
+        if (kind == what) m |= 1u << (i % 32);
+    }
+    return m;
+}
+constexpr uint32_t kQuadZero[3] = {quad_bits(0, 0), quad_bits(1, 0), quad_bits(2, 0)};
+constexpr uint32_t kQuadOne[3] = {quad_bits(0, 1), quad_bits(1, 1), quad_bits(2, 1)};
+constexpr uint32_t kQuadUnit[3] = {quad_bits(0, 2), quad_bits(1, 2), quad_bits(2, 2)};
+static_assert(offsetof(MdnPhysicsParams, rotor_thrust_directions) == 48 &&
+                  offsetof(MdnPhysicsParams, rotor_torque_directions) == 96 &&
+                  offsetof(MdnPhysicsParams, inertia) == 240 && offsetof(MdnPhysicsParams, inertia_inverse) == 276 &&
+                  offsetof(MdnPhysicsParams, gravity_world) == 312 && sizeof(MdnPhysicsParams) == 352,
+              "quad_bits follows the plant's layout");
 // W = wavefronts per workgroup.  W == 1: weights and camera rays are read from
 // global memory (L1/L2 resident).  W > 1: the workgroup stages one copy of the
 // actor first layer, the RAPTOR weights and the camera rays in LDS, shared by
@@ -566,21 +630,44 @@ __global__ __launch_bounds__(64 * W) void rollout_kernel(RolloutArgs a) {
     // the env's state, counters, world and command rows are requested first,
     // so that their latency overlaps the shared weights' staging (a
     // split-tick launch pays this prologue once per tick)
+    // (in a small fleet the wavefront's 64 lanes load each of its envs' words
+    // once, lane l words l, l + 64, ..., and pass them through LDS)
     State s;
     Run r;
-    load_state(a.state, N, nn, s);
-    load_run(a.run, N, nn, r);
     constexpr uint32_t WR = (WORLD_WORDS + G - 1) / G, CMR = (32 + G - 1) / G;
-    float wv[WR], cv[CMR];
+    constexpr uint32_t SE = S ? 4 : 1, SW = S ? 3 : 1;  // small fleet: envs per wavefront, world words per lane
+    static_assert(STATE_WORDS + RW_COUNT <= 64 && WORLD_WORDS <= 192, "a small fleet's words per lane");
+    float wv[S ? 1 : WR], cv[S ? 1 : CMR];
+    float in_w[SE], world_w[SE][SW], cmd_w[SE];
+    const uint32_t wl64 = threadIdx.x % 64, row0 = (threadIdx.x / 64) * EW;  // lane; first LDS row of the wavefront
+    if constexpr (S) {
 #pragma unroll
-    for (uint32_t j = 0; j < WR; j++) {
-        const uint32_t i = lane + G * j;
-        wv[j] = a.world[size_t(nn) * WORLD_WORDS + (i < WORLD_WORDS ? i : 0)];
-    }
+        for (uint32_t e = 0; e < SE; e++) {
+            if (e >= EW) continue;
+            const uint32_t ne = blockIdx.x * EB + row0 + e, ng = ne < N ? ne : 0;
+            const uint32_t i = wl64 < STATE_WORDS + RW_COUNT ? wl64 : 0;
+            in_w[e] = i < STATE_WORDS ? a.state[size_t(i) * N + ng]
+                                      : bits_float(a.run[size_t(i - STATE_WORDS) * N + ng]);
 #pragma unroll
-    for (uint32_t j = 0; j < CMR; j++) {
-        const uint32_t i = lane + G * j;
-        cv[j] = a.commands[size_t(nn) * 32 + (i < 32 ? i : 0)];
+            for (uint32_t j = 0; j < SW; j++) {
+                const uint32_t w = wl64 + 64 * j;
+                world_w[e][j] = a.world[size_t(ng) * WORLD_WORDS + (w < WORLD_WORDS ? w : 0)];
+            }
+            cmd_w[e] = a.commands[size_t(ng) * 32 + wl64 % 32];
+        }
+    } else {
+        load_state(a.state, N, nn, s);
+        load_run(a.run, N, nn, r);
+#pragma unroll
+        for (uint32_t j = 0; j < WR; j++) {
+            const uint32_t i = lane + G * j;
+            wv[j] = a.world[size_t(nn) * WORLD_WORDS + (i < WORLD_WORDS ? i : 0)];
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < CMR; j++) {
+            const uint32_t i = lane + G * j;
+            cv[j] = a.commands[size_t(nn) * 32 + (i < 32 ? i : 0)];
+        }
     }
     __shared__ WeightLds<W, D, SPLIT> s_wt;
     const float* AW1;   // actor W1 transposed [input][hidden]
@@ -620,14 +707,19 @@ __global__ __launch_bounds__(64 * W) void rollout_kernel(RolloutArgs a) {
         WordStage<3 * PIX, 64 * W> st_cam;
         WordStage<ACTOR_TAIL, 64 * W> st_at;
         WordStage<CRITIC_TAIL, 64 * W> st_ct;
-        st_rw.load(a.raptor, threadIdx.x);
-        st_cam.load(a.camera, threadIdx.x);
-        if constexpr (!X) st_at.load(a.actor + HID * D, threadIdx.x);
-        st_ct.load(a.critic + HID * COBS, threadIdx.x);
-        st_rw.store(s_wt.rw, threadIdx.x);
-        st_cam.store(s_wt.cam, threadIdx.x);
-        if constexpr (!X) st_at.store(s_wt.pol, threadIdx.x);
-        st_ct.store(s_wt.pol + ACTOR_TAIL, threadIdx.x);
+        const bool policy = !S || acts, camera = !S || casts;  // (a large fleet's launches nearly all do both)
+        if (policy) st_rw.load(a.raptor, threadIdx.x);
+        if (camera) st_cam.load(a.camera, threadIdx.x);
+        if (policy) {
+            if constexpr (!X) st_at.load(a.actor + HID * D, threadIdx.x);
+            st_ct.load(a.critic + HID * COBS, threadIdx.x);
+            st_rw.store(s_wt.rw, threadIdx.x);
+        }
+        if (camera) st_cam.store(s_wt.cam, threadIdx.x);
+        if (policy) {
+            if constexpr (!X) st_at.store(s_wt.pol, threadIdx.x);
+            st_ct.store(s_wt.pol + ACTOR_TAIL, threadIdx.x);
+        }
         __syncthreads();
         if constexpr (!X) {  // the action noise scales are fixed for the launch
             if (threadIdx.x < 8) {
@@ -674,12 +766,33 @@ __global__ __launch_bounds__(64 * W) void rollout_kernel(RolloutArgs a) {
     __shared__ float s_rh[W > 1 ? E : 1][17];
 
     float* world = s_world[grp];
+    if constexpr (S) {
+        static_assert(OS >= 64, "the observation row passes the state and counters");
 #pragma unroll
-    for (uint32_t j = 0; j < WR; j++)
-        if (lane + G * j < WORLD_WORDS) world[lane + G * j] = wv[j];
+        for (uint32_t e = 0; e < SE; e++) {
+            if (e >= EW) continue;
+            s_obs[row0 + e][wl64] = in_w[e];
 #pragma unroll
-    for (uint32_t j = 0; j < CMR; j++)
-        if (lane + G * j < 32) s_cmd[grp][lane + G * j] = cv[j];
+            for (uint32_t j = 0; j < SW; j++)
+                if (wl64 + 64 * j < WORLD_WORDS) s_world[row0 + e][wl64 + 64 * j] = world_w[e][j];
+            if (wl64 < 32) s_cmd[row0 + e][wl64] = cmd_w[e];
+        }
+        group_sync();
+        float* sd = &s.p[0];
+        uint32_t* rd = reinterpret_cast<uint32_t*>(&r);
+#pragma unroll
+        for (uint32_t i = 0; i < STATE_WORDS; i++) sd[i] = s_obs[grp][i];
+#pragma unroll
+        for (uint32_t i = 0; i < RW_COUNT; i++) rd[i] = float_bits(s_obs[grp][STATE_WORDS + i]);
+        for (uint32_t c = lane; c < 16; c += G) s_rh[grp][c] = s_obs[grp][STATE_WORDS + RW_HIDDEN + c];
+    } else {
+#pragma unroll
+        for (uint32_t j = 0; j < WR; j++)
+            if (lane + G * j < WORLD_WORDS) world[lane + G * j] = wv[j];
+#pragma unroll
+        for (uint32_t j = 0; j < CMR; j++)
+            if (lane + G * j < 32) s_cmd[grp][lane + G * j] = cv[j];
+    }
     {   // pooled ring cache: LDS slot f%K holds frame f for the last K frames
         // (a launch that begins at act already holds the frame cast for the
         // current step, if one was due); the 2x2 minima of the group's
@@ -688,7 +801,31 @@ __global__ __launch_bounds__(64 * W) void rollout_kernel(RolloutArgs a) {
                          : r.steps == 0                         ? -1
                                                                 : int((r.steps - 1) / C.sensor_period);
         constexpr uint32_t RC = (uint32_t(K) * POOL + G - 1) / G, CH = 10;  // cells per lane; per round
-        for (uint32_t c0 = 0; c0 < (casts ? RC : 0u); c0 += CH) {
+        if constexpr (S) {  // one env at a time over the wavefront, each row pair of a cell one 8-byte load
+            constexpr uint32_t SC = (uint32_t(K) * POOL + 63) / 64;
+            for (uint32_t e = 0; e < (casts ? EW : 0u); e++) {
+                const int last_e = __builtin_amdgcn_readlane(last, e * G);
+                const uint32_t ne = blockIdx.x * EB + row0 + e;
+                if (ne >= N) break;
+                float2 px[SC][2];
+#pragma unroll
+                for (uint32_t c = 0; c < SC; c++) {
+                    const uint32_t cell = min(wl64 + 64 * c, uint32_t(K) * POOL - 1), b = cell % POOL;
+                    const float* src = a.sensors + (size_t(ne) * 8 + (uint32_t(last_e - int(cell / POOL)) & 7u)) * PIX +
+                                       (b / 10) * 40 + (b % 10) * 2;
+                    px[c][0] = *reinterpret_cast<const float2*>(src);
+                    px[c][1] = *reinterpret_cast<const float2*>(src + 20);
+                }
+#pragma unroll
+                for (uint32_t c = 0; c < SC; c++) {
+                    const uint32_t cell = wl64 + 64 * c;
+                    if (cell >= uint32_t(K) * POOL) continue;
+                    const float m = min_f(min_f(min_f(min_f(12.0f, px[c][0].x), px[c][0].y), px[c][1].x), px[c][1].y);
+                    s_ring[row0 + e][(uint32_t(last_e - int(cell / POOL)) % uint32_t(K)) * POOL + cell % POOL] = m;
+                }
+            }
+        }
+        for (uint32_t c0 = 0; c0 < (casts && !S ? RC : 0u); c0 += CH) {
             float px[CH][4];
 #pragma unroll
             for (uint32_t c = 0; c < CH; c++) {
@@ -721,7 +858,7 @@ __global__ __launch_bounds__(64 * W) void rollout_kernel(RolloutArgs a) {
     float hu[U];
 #pragma unroll
     for (int j = 0; j < U; j++) hu[j] = bits_float(a.run[size_t(RW_HIDDEN + lane + G * j) * N + nn]);
-    if constexpr (W > 1) {
+    if constexpr (W > 1 && !S) {
         constexpr uint32_t HR = (16 + G - 1) / G;
         float hv[HR];
 #pragma unroll
@@ -740,9 +877,11 @@ __global__ __launch_bounds__(64 * W) void rollout_kernel(RolloutArgs a) {
     // W > 1: the policy tails from LDS and the critic's first layer in
     // registers (the tick loop then reads no weights from global memory)
     float cw1[TileMap<S>::NT][COBS / 4];
-    if constexpr (W > 1) critic_operands<COBS, S>(EB, a.critic_w1t, cw1);
+    if constexpr (W > 1)
+        if (!S || acts) critic_operands<COBS, S>(EB, a.critic_w1t, cw1);
     RaptorRegs rops;
-    if constexpr (W > 1) raptor_operands(RW, rops);
+    if constexpr (W > 1)
+        if (!S || acts) raptor_operands(RW, rops);
     const float* AT = A + a_b1;
     const float* CT = CR + c_b1;
     if constexpr (W > 1) {
@@ -756,16 +895,26 @@ __global__ __launch_bounds__(64 * W) void rollout_kernel(RolloutArgs a) {
     constexpr uint32_t PW = sizeof(MdnPhysicsParams) / 4;
     __shared__ float s_ep[DYN ? E : 1][DYN ? PW : 1];
     __shared__ PhysRecip s_erp[DYN ? E : 1];
+    bool plants_quad = true;  // every plant of the wavefront has the standard structure (derivative_quad)
     if constexpr (DYN) {
-        const float* src = reinterpret_cast<const float*>(a.env_phys + nn);
-        constexpr uint32_t PR = (PW + G - 1) / G;
-        float pv[PR];
+        if (acts) {
+            const float* src = reinterpret_cast<const float*>(a.env_phys + nn);
+            constexpr uint32_t PR = PW / G;
+            static_assert(PW % G == 0 && G == 8, "whole plant words per lane");
+            float pv[PR];
 #pragma unroll
-        for (uint32_t j = 0; j < PR; j++) pv[j] = src[lane + G * j < PW ? lane + G * j : 0];
+            for (uint32_t j = 0; j < PR; j++) pv[j] = src[lane + G * j];
 #pragma unroll
-        for (uint32_t j = 0; j < PR; j++)
-            if (lane + G * j < PW) s_ep[grp][lane + G * j] = pv[j];
-        if (lane == 0) s_erp[grp] = phys_recip(a.env_phys[nn]);
+            for (uint32_t j = 0; j < PR; j++) {
+                s_ep[grp][lane + G * j] = pv[j];
+                const uint32_t sh = lane + G * (j % 4), u = float_bits(pv[j]);  // bit of word lane + G j
+                plants_quad = plants_quad && (!((kQuadZero[j / 4] >> sh) & 1u) || u == 0u) &&
+                              (!((kQuadOne[j / 4] >> sh) & 1u) || u == 0x3f800000u) &&
+                              (!((kQuadUnit[j / 4] >> sh) & 1u) || (u & 0x7fffffffu) == 0x3f800000u);
+            }
+            plants_quad = __all(plants_quad);
+            if (lane == 0) s_erp[grp] = phys_recip(a.env_phys[nn]);
+        }
     }
     group_sync();
 
@@ -1419,7 +1568,8 @@ __global__ __launch_bounds__(64 * W) void rollout_kernel(RolloutArgs a) {
         const float wind[3] = {world[166] * EP.mass, world[167] * EP.mass, world[168] * EP.mass};
         // the standard-structure derivative takes wind / mass, the same
         // division physics.hpp:101 repeats in every derivative evaluation
-        const float wm[3] = {div_r(wind[0], RP.mass), div_r(wind[1], RP.mass), div_r(wind[2], RP.mass)};
+        const double rmass = DYN ? s_erp[DYN ? grp : 0].mass : RP.mass;
+        const float wm[3] = {div_r(wind[0], rmass), div_r(wind[1], rmass), div_r(wind[2], rmass)};
         bool nzero = no_negative_zero(s);  // no component of s is -0 (derivative_quad's condition)
         for (uint32_t step = 0; step < C.substeps; step++) {
             float mo[22] = {0};
@@ -1451,8 +1601,10 @@ __global__ __launch_bounds__(64 * W) void rollout_kernel(RolloutArgs a) {
 #pragma unroll
                 for (int q = 0; q < 4; q++) r.motors[q] = act[q];
                 State nx;
-                if constexpr (DYN) physics_step(EP, s_erp[grp], s, act, wind, nx);
-                else if ((CF || a.quad) && !__any(!nzero)) physics_step<true>(P, RP, s, act, wm, nx);
+                if constexpr (DYN) {
+                    if (plants_quad && !__any(!nzero)) physics_step<true>(EP, s_erp[grp], s, act, wm, nx);
+                    else physics_step(EP, s_erp[grp], s, act, wind, nx);
+                } else if ((CF || a.quad) && !__any(!nzero)) physics_step<true>(P, RP, s, act, wm, nx);
                 else physics_step(P, RP, s, act, wind, nx);
                 // every component finite (isfinite_f) and none -0, in integer
                 // form: the largest exponent field and the smallest bits ^ sign
@@ -1639,7 +1791,22 @@ __global__ __launch_bounds__(64 * W) void rollout_kernel(RolloutArgs a) {
 #pragma unroll
         for (int c = 0; c < 16; c++) r.hidden[c] = s_rh[grp][c];
     }
-    if (live) {
+    if constexpr (S) {  // through LDS, lane l storing word l of each env
+        const float* sd = &s.p[0];
+        const uint32_t* rd = reinterpret_cast<const uint32_t*>(&r);
+#pragma unroll
+        for (uint32_t i = 0; i < STATE_WORDS; i++) s_obs[grp][i] = sd[i];
+#pragma unroll
+        for (uint32_t i = 0; i < RW_COUNT; i++) s_obs[grp][STATE_WORDS + i] = bits_float(rd[i]);
+        group_sync();
+        for (uint32_t e = 0; e < EW; e++) {
+            const uint32_t ne = blockIdx.x * EB + row0 + e;
+            if (ne >= N || wl64 >= STATE_WORDS + RW_COUNT) continue;
+            const float v = s_obs[row0 + e][wl64];
+            if (wl64 < STATE_WORDS) a.state[size_t(wl64) * N + ne] = v;
+            else a.run[size_t(wl64 - STATE_WORDS) * N + ne] = float_bits(v);
+        }
+    } else if (live) {
         store_state(a.state, N, n, s, lane, G);
         store_run(a.run, N, n, r, lane, G);
     }

@@ -67,6 +67,33 @@ def test_fleet_plants_and_tasks(n, delay, obs):
     _collect_both(sim, ora, 6, ["environment_physics", "task_states"])
 
 
+def test_fleet_plants_of_any_structure():
+    """Per-episode plants the host uploads: standard structure in some
+    wavefronts (the specialised derivative), a tilted rotor, an off-diagonal
+    inertia or a -0 in others (the general one)."""
+    say("case: uploaded plants, standard and not")
+    cfg = config(n=48, family=1, seed=4, speed=1.0, distance=3.0, max_steps=400)
+    sim, _, ora = make_pair(cfg, 6)
+    rt = task_runtime(1.0)
+    for x in (sim, ora):
+        x.set_runtime(rt)
+        x.set("actor", sim.get("actor"))
+        x.set("critic", sim.get("critic"))
+        x.reset()
+    plants = sim.get("environment_physics")
+    plants["rotor_thrust_directions"][5, 3:6] = [0.1, 0.0, 0.99]
+    plants["inertia"][11, 1] = 1e-7
+    plants["rotor_positions"][17, 2] = -0.0
+    plants["gravity_world"][23, 0] = 0.5
+    plants["rotor_torque_directions"][29, 2] = 0.9
+    for x in (sim, ora):
+        x.set("environment_physics", plants)
+        x.collect(6)
+    sim.sync()
+    bad = compare(sim, ora, ENV_BUFFERS + ROW_BUFFERS + ["environment_physics"])
+    assert not bad, bad
+
+
 @pytest.mark.parametrize("n", [2048, 2049])
 def test_memory_workgroups(n):
     say("case: geometry memory, fleet of", n)
