@@ -21,41 +21,172 @@ using namespace mdn;
 constexpr float LOG_TWO_PI = 1.8378770664093453f;
 constexpr uint32_t MAX_IN = 1024, MAX_HIDDEN = 8192;
 
-// One workgroup per row: the row's inputs in LDS, hidden units strided over
-// the 256 threads, then one thread per output (means, or the value) runs the
-// output chain over the hidden units in order.  Layouts (ppo.hpp:35-45):
-// W1[H][D] at 0, b1[H], W2[O][H], b2[O]; the actor (O = 4) then has
-// log_std[4], the critic (O = 1) nothing.
-__global__ __launch_bounds__(256) void mlp_forward_kernel(const float* __restrict__ w, const float* __restrict__ x,
-                                                          uint32_t D, uint32_t H, uint32_t O, uint32_t prior,
-                                                          uint64_t B, float* __restrict__ hidden,
-                                                          float* __restrict__ out) {
-    __shared__ float s_x[MAX_IN];
-    __shared__ float s_h[MAX_HIDDEN];
-    const uint64_t row = blockIdx.x;
-    if (row >= B) return;  // the whole workgroup leaves together
-    const uint32_t t = threadIdx.x;
-    const float* xr = x + row * D;
-    for (uint32_t i = t; i < D; i += 256) s_x[i] = xr[i];
-    __syncthreads();
+// First layer of 16 rows x 64 hidden units per workgroup on the matrix cores:
+// each of the four wavefronts owns 16 units, and one 16x16x4 step is the same
+// chain of fused multiply-adds, bias first and inputs ascending, as the scalar
+// form.  Layouts (ppo.hpp:35-45): W1[H][D] at 0, b1[H], W2[O][H], b2[O]; the
+// actor (O = 4) then has log_std[4], the critic (O = 1) nothing.
+//
+// Bound by latency: a batch of 4,096 rows is one workgroup per CU, so a tile
+// loads its 80 rows of up to 192 inputs (60 loads a lane, coalesced, all in
+// flight together) and then runs 46 dependent steps.  LDS rows are 196 words
+// apart: the 16 rows x 4 inputs that a step reads lie in 64 different banks.
+// Inputs beyond D multiply 0 by -0, which changes no partial sum.  184 -> 64
+// -> 4 with the output chains: 9.7 us at 4,096 rows, 6.8 at one (one workgroup
+// per row with scalar chains over uncoalesced weight rows: 29.6 and 13.3).
+//
+// O > 0: the whole hidden layer is this tile (H <= 64) and its output chains
+// run here.  O = 0: wider layers; output_kernel follows.
+constexpr uint32_t ROWS = 16, UNITS = 64, SLAB = 192, STRIDE = SLAB + 4, HSTRIDE = UNITS + 4;
+using f32x4 = float __attribute__((ext_vector_type(4)));
+
+template <uint32_t O>
+__global__ __launch_bounds__(256) void hidden_kernel(const float* __restrict__ w, const float* __restrict__ x,
+                                                     uint32_t D, uint32_t H, uint32_t prior, uint64_t B,
+                                                     float* __restrict__ hidden, float* __restrict__ out) {
+    __shared__ float s_w[UNITS * STRIDE];
+    __shared__ float s_x[ROWS * STRIDE];
+    __shared__ __align__(16) float s_h[O ? ROWS * HSTRIDE : 4];
+    __shared__ __align__(16) float s_w2[O ? O * HSTRIDE : 4];
+    const uint32_t t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const uint64_t row0 = uint64_t(blockIdx.x) * ROWS;
+    const uint32_t unit0 = blockIdx.y * UNITS;
     const float* b1 = w + size_t(H) * D;
-    for (uint32_t h = t; h < H; h += 256) {
-        const float* wr = w + size_t(h) * D;
-        float z = b1[h];
-        for (uint32_t i = 0; i < D; i++) z = fma_f(wr[i], s_x[i], z);
+    const uint32_t unit = unit0 + wave * 16 + (lane & 15);
+    const float bias = unit < H ? b1[unit] : 0.0f;
+    if constexpr (O != 0) {
+        if (t < O * UNITS) {
+            const uint32_t o = t / UNITS, h = t % UNITS;
+            s_w2[o * HSTRIDE + h] = h < H ? b1[H + size_t(o) * H + h] : -0.0f;
+        }
+    }
+    f32x4 acc = {bias, bias, bias, bias};
+    for (uint32_t k0 = 0; k0 < D; k0 += SLAB) {
+        const uint32_t kn = D - k0 < SLAB ? D - k0 : SLAB;
+        float rw[UNITS / 4][SLAB / 64], rx[ROWS / 4][SLAB / 64];
+#pragma unroll
+        for (uint32_t r = 0; r < UNITS / 4; r++) {
+            const uint32_t u = unit0 + wave + 4 * r;
+#pragma unroll
+            for (uint32_t c = 0; c < SLAB / 64; c++) {
+                const uint32_t k = lane + 64 * c;
+                rw[r][c] = u < H && k < kn ? w[size_t(u) * D + k0 + k] : -0.0f;
+            }
+        }
+#pragma unroll
+        for (uint32_t r = 0; r < ROWS / 4; r++) {
+            const uint64_t row = row0 + wave + 4 * r;
+#pragma unroll
+            for (uint32_t c = 0; c < SLAB / 64; c++) {
+                const uint32_t k = lane + 64 * c;
+                rx[r][c] = row < B && k < kn ? x[row * D + k0 + k] : 0.0f;
+            }
+        }
+        if (k0) __syncthreads();  // the last slab has been read
+#pragma unroll
+        for (uint32_t c = 0; c < SLAB / 64; c++) {
+#pragma unroll
+            for (uint32_t r = 0; r < UNITS / 4; r++) s_w[(wave + 4 * r) * STRIDE + lane + 64 * c] = rw[r][c];
+#pragma unroll
+            for (uint32_t r = 0; r < ROWS / 4; r++) s_x[(wave + 4 * r) * STRIDE + lane + 64 * c] = rx[r][c];
+        }
+        __syncthreads();
+        const float* fx = s_x + (lane & 15) * STRIDE + (lane >> 4);
+        const float* fw = s_w + (wave * 16 + (lane & 15)) * STRIDE + (lane >> 4);
+#pragma unroll 8
+        for (uint32_t k = 0; k < kn; k += 4) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(fx[k], fw[k], acc, 0, 0, 0);
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < 4; r++) {
+        const float z = acc[r];
         const float a = tanh_f(z);
-        s_h[h] = a;
-        if (hidden) hidden[row * H + h] = a;
+        const uint32_t m = 4 * (lane >> 4) + r;
+        if (unit < H && row0 + m < B) hidden[(row0 + m) * H + unit] = a;
+        if constexpr (O != 0) s_h[m * HSTRIDE + wave * 16 + (lane & 15)] = unit < H ? a : 0.0f;
     }
-    __syncthreads();
-    if (t < O) {
-        const float* w2 = b1 + H + size_t(t) * H;
-        float z = b1[H + size_t(O) * H + t];
-        for (uint32_t h = 0; h < H; h++) z = fma_f(w2[h], s_h[h], z);
-        // geometry prior (ppo.hpp:30-34, 77): the hint inputs join the first three means
-        if (prior && t < 3) z += s_x[D - 3 + t];
-        out[row * O + t] = z;
+    if constexpr (O != 0) {
+        __syncthreads();
+        const uint32_t m = t / O, o = t % O;
+        if (m < ROWS && row0 + m < B) {
+            float z = b1[H + size_t(O) * H + o];
+            const f32x4* h4 = reinterpret_cast<const f32x4*>(s_h + m * HSTRIDE);
+            const f32x4* v4 = reinterpret_cast<const f32x4*>(s_w2 + o * HSTRIDE);
+#pragma unroll
+            for (uint32_t q = 0; q < UNITS / 4; q++) {
+                const f32x4 h = h4[q], v = v4[q];
+#pragma unroll
+                for (uint32_t i = 0; i < 4; i++) z = fma_f(v[i], h[i], z);
+            }
+            // geometry prior (ppo.hpp:30-34, 77): the hint inputs join the first three means
+            if (prior && o < 3) z += x[(row0 + m) * D + D - 3 + o];
+            out[(row0 + m) * O + o] = z;
+        }
     }
+}
+
+// Output chains over a hidden layer wider than one tile: one wavefront runs
+// the 16 rows x O chains of a workgroup, all four bring the next 256 units of
+// the rows and of W2 while it does.  Bound by the chain itself, about 6 cycles
+// a unit.  184 -> 2,048 -> 4 at 1,024 rows: hidden layer 28.7 us, this 14.8
+// (scalar chains: 238 together).  A layer of one tile stays with the fused
+// form: a second launch costs more than its chain of 64.
+constexpr uint32_t OUT_SLAB = 256, OUT_STRIDE = OUT_SLAB + 4;
+
+template <uint32_t O>
+__global__ __launch_bounds__(256) void output_kernel(const float* __restrict__ w, const float* __restrict__ x,
+                                                     uint32_t D, uint32_t H, uint32_t prior, uint64_t B,
+                                                     const float* __restrict__ hidden, float* __restrict__ out) {
+    __shared__ __align__(16) float s_h[2][ROWS * OUT_STRIDE];
+    __shared__ __align__(16) float s_v[2][O * OUT_STRIDE];
+    const uint32_t t = threadIdx.x, m = t / O, o = t % O;
+    const uint64_t row0 = uint64_t(blockIdx.x) * ROWS;
+    const float* w2 = w + size_t(H) * D + H;
+    const bool mine = m < ROWS && row0 + m < B;
+    float rh[ROWS], rv[O];
+    auto load = [&](uint32_t h0) {
+        const bool in = h0 + t < H;
+#pragma unroll
+        for (uint32_t r = 0; r < ROWS; r++) rh[r] = in && row0 + r < B ? hidden[(row0 + r) * H + h0 + t] : 0.0f;
+#pragma unroll
+        for (uint32_t r = 0; r < O; r++) rv[r] = in ? w2[size_t(r) * H + h0 + t] : -0.0f;
+    };
+    load(0);
+    float z = mine ? w2[size_t(O) * H + o] : 0.0f;
+    for (uint32_t h0 = 0, b = 0; h0 < H; h0 += OUT_SLAB, b ^= 1) {
+#pragma unroll
+        for (uint32_t r = 0; r < ROWS; r++) s_h[b][r * OUT_STRIDE + t] = rh[r];
+#pragma unroll
+        for (uint32_t r = 0; r < O; r++) s_v[b][r * OUT_STRIDE + t] = rv[r];
+        __syncthreads();  // also: every wavefront is past the slab before the last, whose buffer comes next
+        if (h0 + OUT_SLAB < H) load(h0 + OUT_SLAB);
+        if (mine) {
+            const f32x4* h4 = reinterpret_cast<const f32x4*>(s_h[b] + m * OUT_STRIDE);
+            const f32x4* v4 = reinterpret_cast<const f32x4*>(s_v[b] + o * OUT_STRIDE);
+#pragma unroll 8
+            for (uint32_t q = 0; q < OUT_SLAB / 4; q++) {
+                const f32x4 h = h4[q], v = v4[q];
+#pragma unroll
+                for (uint32_t i = 0; i < 4; i++) z = fma_f(v[i], h[i], z);
+            }
+        }
+    }
+    if (mine) {
+        if (prior && o < 3) z += x[(row0 + m) * D + D - 3 + o];  // geometry prior (ppo.hpp:30-34, 77)
+        out[(row0 + m) * O + o] = z;
+    }
+}
+
+template <uint32_t O>
+hipError_t launch_forward(const float* w, const float* x, uint32_t D, uint32_t H, uint32_t prior, uint64_t B,
+                          float* hidden, float* out, hipStream_t st) {
+    const dim3 tiles(uint32_t((B + ROWS - 1) / ROWS), (H + UNITS - 1) / UNITS);
+    if (H <= UNITS) {
+        hipLaunchKernelGGL(hidden_kernel<O>, tiles, dim3(256), 0, st, w, x, D, H, prior, B, hidden, out);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(hidden_kernel<0>, tiles, dim3(256), 0, st, w, x, D, H, prior, B, hidden, out);
+    hipLaunchKernelGGL(output_kernel<O>, dim3(tiles.x), dim3(256), 0, st, w, x, D, H, prior, B, hidden, out);
+    return hipGetLastError();
 }
 
 __device__ __forceinline__ float log_prob(const float* a, const float* m, const float* ls) {
@@ -141,12 +272,11 @@ extern "C" {
 hipError_t fppo_launch_forward(const float* w, const float* x, uint32_t D, uint32_t H, uint32_t O, uint32_t prior,
                                uint64_t B, float* hidden, float* out, hipStream_t st) {
     if (B == 0) return hipSuccess;
-    if (D == 0 || D > fppo::MAX_IN || H == 0 || H > fppo::MAX_HIDDEN || O == 0 || O > 256 || B > 0x7fffffffull ||
-        (prior && D < 3))
+    if (D == 0 || D > fppo::MAX_IN || H == 0 || H > fppo::MAX_HIDDEN || (O != 1 && O != 4) || !hidden ||
+        B > 0x7fffffffull || (prior && D < 3))
         return hipErrorInvalidValue;
-    hipLaunchKernelGGL(fppo::mlp_forward_kernel, dim3(uint32_t(B)), dim3(256), 0, st, w, x, D, H, O, prior, B, hidden,
-                       out);
-    return hipGetLastError();
+    return O == 4 ? fppo::launch_forward<4>(w, x, D, H, prior, B, hidden, out, st)
+                  : fppo::launch_forward<1>(w, x, D, H, prior, B, hidden, out, st);
 }
 
 hipError_t fppo_launch_log_prob(const float* act, const float* mean, const float* log_std, uint32_t ls_stride,

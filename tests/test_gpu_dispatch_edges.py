@@ -172,3 +172,38 @@ def test_normalize_sizes(count):
         assert hip.hipFree(dev) == 0
         assert np.array_equal(host[offset:offset + count], want), offset
         assert np.all(host[:offset] == 7.0) and np.all(host[offset + count:] == 7.0)
+
+
+def _mlp(d, h, b, seed, special):
+    rng = np.random.default_rng(seed)
+    w = rng.normal(0, 0.3, h * d + h + 4 * h + 8).astype(np.float32)
+    x = rng.uniform(-1, 1, (b, d)).astype(np.float32)
+    if special:  # signed zeros, subnormals, infinities and NaN in inputs and weights
+        x.flat[::7] = -0.0
+        x.flat[3::11] = 1e-41
+        w[5::13] = -0.0
+        w[2::17] = 3e-42
+        if b > 2:
+            x[1, d // 2] = np.inf
+            x[2, d - 1] = np.nan
+    return w, x
+
+
+@pytest.mark.parametrize("special", [0, 1])
+@pytest.mark.parametrize("d,h,b", [(1, 1, 1), (2, 5, 3), (4, 64, 16), (181, 64, 17), (184, 63, 33), (191, 65, 15),
+                                   (193, 128, 31), (192, 256, 16), (385, 257, 20), (824, 320, 18), (1024, 512, 1)])
+def test_forward_sizes(d, h, b, special):
+    say("case: forward,", b, "rows", d, "inputs", h, "units, special", special)
+    w, x = _mlp(d, h, b, d + h + b, special)
+    ho, mo = np.zeros((b, h), np.float32), np.zeros((b, 4), np.float32)
+    oracle().orc_actor_forward_batch(ptr(w), ptr(x), d, h, b, ptr(ho), ptr(mo))
+    if d == 824:  # the oracle adds the hint at 184 inputs only
+        mo[:, :3] += x[:, -3:]
+    hid, mean = ops.actor_forward(w, x, hidden_dim=h)
+    assert np.array_equal(hid, ho, equal_nan=True) and np.array_equal(mean, mo, equal_nan=True)
+    if d in (184, 824):
+        return  # a critic has no hint to add
+    # a critic whose output row is the actor's first
+    c = np.concatenate([w[:h * d + 2 * h], w[h * d + 5 * h:h * d + 5 * h + 1]])
+    hid, value = ops.critic_forward(c, x, hidden_dim=h)
+    assert np.array_equal(hid, ho, equal_nan=True) and np.array_equal(value, mo[:, 0], equal_nan=True)
