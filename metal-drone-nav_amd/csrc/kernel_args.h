@@ -168,10 +168,10 @@ struct MbArgs {
     float* grad;  // P_TOTAL: actor, critic, metric sums
 };
 constexpr uint32_t MB_REC_WORDS = 4 * 256 * 64 + 256 * 16;
-// Most chunks that path takes.  Us per step of one Adam step's kernels, this
-// path and the chunk kernel: 20 and 68 at 2 chunks, 33 and 77 at 16, 65 and
-// 83 at 64, 84 and 85 at 96, 103 and 86 at 128 (its records and their re-reads
-// go through L2, where the chunk kernel keeps them in LDS).
+// Most chunks that path takes.  Us per Adam step, this path: 19 at 2 chunks,
+// 27 at 16, 62 at 64, 73 at 80, 83 at 96, 103 at 128; the chunk kernel: 68 at
+// 2, 77 at 16, 74 from 80 to 128 (this path's records and their re-reads go
+// through L2, where the chunk kernel keeps them in LDS).
 constexpr uint32_t MB_MAX_CHUNKS = 80;
 constexpr uint32_t CHUNK_ROWS = 256;  // rows of one gradient chunk
 

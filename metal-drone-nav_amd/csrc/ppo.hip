@@ -527,6 +527,7 @@ __global__ __launch_bounds__(256) void norm_apply_kernel(float* __restrict__ a, 
 // which leaves every accumulator (including -0.0) unchanged.
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef float v4f __attribute__((ext_vector_type(4)));
+typedef float v2f __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ v16f mfma32(float a, float b, v16f c) {
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
@@ -1098,162 +1099,237 @@ __global__ __launch_bounds__(256) void chunk_reduce_kernel(const float* __restri
 // gradient needs no chunk reduction.
 constexpr uint32_t MB_HA = 0, MB_DA = 256 * 64, MB_HC = 2 * 256 * 64, MB_DC = 3 * 256 * 64, MB_RS = 4 * 256 * 64;
 constexpr uint32_t MB_FWD_ROWS = 16;
+// Positions in the forward's LDS tiles.  A lane of a 16x16x4 step takes the
+// input 4 step + l/16 of row or unit l % 16.  Each 16 inputs are stored by
+// that remainder first, so the inputs of a lane's four consecutive steps are
+// one 16-byte read; the last 8 of the 184 by pairs.  The row strides are four
+// times an odd number, which spreads 16 rows' reads over all banks.
+constexpr uint32_t MB_KP = 184, MB_WS = 188, MB_CS = 36, MB_HS = 20;
+__device__ __forceinline__ uint32_t mb_pos(uint32_t k) {
+    return k < 176 ? (k & ~15u) + 4 * (k % 4) + (k % 16) / 4 : 176 + 2 * (k % 4) + (k - 176) / 4;
+}
+// 16 rows per workgroup: a chain of dependent phases in few wavefronts, each
+// bound by latency.  Per workgroup at 181 inputs, in cycles: 3.0 k until the
+// last load is issued, 1.4 k to lay the tiles out in LDS, 3.6 k for the first
+// layer (46 dependent steps at 50) with its activations, 0.9 k for the means,
+// 2.0 k for the objective, 1.0 k for the deltas.  Address arithmetic without
+// divisions, four steps' operands per LDS read, padding in the tiles instead
+// of selects in the chain, the scale factors beside the layers, the objective
+// in a wavefront that is idle before it, and records written four units at a
+// time by wavefronts that read the rest ahead: 14.6 -> 12.9 k cycles, the
+// kernel 7.2 -> 6.5 us for 256 rows.
 template <uint32_t D, bool ONE>
 __global__ __launch_bounds__(512) void mb_forward_kernel(MbArgs m) {
     using L = AL<D>;
     const RowArgs& a = m.r;
-    constexpr uint32_t XS = D | 1u, WS = HID + 1;  // odd strides: rows fall in distinct banks
-    __shared__ float s_w[D * WS];                  // actor W1^T [input][unit]
-    __shared__ float s_cw[COBS * WS];              // critic W1^T
-    __shared__ float s_t[5 * HID + 8 + 2 * HID + 1];  // actor b1, W2, b2, log_std; critic b1, w2, b2
-    __shared__ float s_x[MB_FWD_ROWS][XS];
-    __shared__ float s_c[MB_FWD_ROWS][COBS + 1];
-    __shared__ float s_ha[MB_FWD_ROWS][HID + 1];
-    __shared__ float s_hc[MB_FWD_ROWS][HID + 1];
+    static_assert(D > 128 && D <= MB_KP && COBS == 32 && HID == 64 && MB_FWD_ROWS == 16, "staging map");
+    constexpr uint32_t AT = 5 * HID + 8;  // actor tail words from b1 on
+    __shared__ __attribute__((aligned(16))) float s_w[HID * MB_WS];           // actor W1 [unit][mb_pos]
+    __shared__ __attribute__((aligned(16))) float s_cw[HID * MB_CS];          // critic W1
+    __shared__ __attribute__((aligned(16))) float s_t[AT + 2 * HID + 1];      // actor b1, W2, b2, log_std; critic b1, w2, b2
+    __shared__ __attribute__((aligned(16))) float s_x[MB_FWD_ROWS * MB_WS];   // inputs [row][mb_pos]
+    __shared__ __attribute__((aligned(16))) float s_c[MB_FWD_ROWS * MB_CS];
     __shared__ float s_mv[MB_FWD_ROWS][5];   // means, value
-    __shared__ float s_rs[MB_FWD_ROWS][16];  // d mean, d log_std, metric terms, d value
+    __shared__ __attribute__((aligned(16))) float s_rs[MB_FWD_ROWS][16];  // d mean, d log_std, metric terms, d value
     __shared__ float s_ex[8];                 // row_scale_exp
-    const uint32_t t = threadIdx.x, wv = t / 64, l = t % 64;
+    const uint32_t t = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(t / 64), l = t % 64;
     const uint32_t n0 = blockIdx.x * MB_FWD_ROWS;
     const uint32_t live_rows = a.b - n0 < MB_FWD_ROWS ? a.b - n0 : MB_FWD_ROWS;
     float* rec = m.rec + (ONE ? 0 : size_t(n0 / CHUNK) * MB_REC_WORDS);  // this chunk's records
-    constexpr uint32_t AT = 5 * HID + 8;  // actor tail words from b1 on
-    float* s_at = s_t;
-    float* s_ct = s_t + AT;
+    const float* s_at = s_t;
+    const float* s_ct = s_t + AT;
     float ract[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-    float rolp = 0.0f, radv = 0.0f, rret = 0.0f;
-    {   // every load of the staging issued before any store
-        constexpr uint32_t NW = (D * HID + 511) / 512, NCW = COBS * HID / 512, NX = (MB_FWD_ROWS * D + 511) / 512;
-        float w[NW], cw[NCW], xv[NX], cv, tv[2];
-        // the first layers from the flat vectors ([unit][input]), transposed
-        // into LDS (the transposed copies are refreshed once per update)
+    float rolp = 0.0f, radv = 0.0f, rret = 0.0f, nmean = 0.0f, ninv = 1.0f;
+    {   // every load of the staging issued before any store: wavefront wv takes
+        // units 8 wv .. 8 wv + 7 and rows 2 wv, 2 wv + 1, a lane the inputs
+        // l, l + 64 and l + 128
+        // (out-of-range ones read a clamped place and are replaced, which keeps
+        // the loads free of branches)
+        constexpr uint32_t NU = HID / 8, NR = MB_FWD_ROWS / 8;
+        const bool last = l < D - 128;
+        const uint32_t l2 = last ? l + 128 : D - 1;
+        float w[NU][3], xv[NR][3], cw[4], cv, tv[2];
+        const float* wg = a.actor + wv * NU * D;  // the flat vector's [unit][input]
 #pragma unroll
-        for (uint32_t k = 0; k < NW; k++) {
-            const uint32_t e = t + 512 * k;
-            w[k] = e < D * HID ? a.actor[e] : 0.0f;
+        for (uint32_t u = 0; u < NU; u++) {
+            w[u][0] = wg[u * D + l];
+            w[u][1] = wg[u * D + l + 64];
+            w[u][2] = wg[u * D + l2];
         }
 #pragma unroll
-        for (uint32_t k = 0; k < NCW; k++) cw[k] = a.critic[t + 512 * k];
+        for (uint32_t k = 0; k < 4; k++) cw[k] = a.critic[t + 512 * k];
 #pragma unroll
-        for (uint32_t k = 0; k < NX; k++) {
-            const uint32_t e = t + 512 * k, r = e / D;
-            xv[k] = e < MB_FWD_ROWS * D && r < live_rows ? a.obs[size_t(n0) * D + e] : 0.0f;
+        for (uint32_t u = 0; u < NR; u++) {
+            const uint32_t r = wv * NR + u < live_rows ? wv * NR + u : 0;
+            const float* xg = a.obs + size_t(n0 + r) * D;
+            xv[u][0] = xg[l];
+            xv[u][1] = xg[l + 64];
+            xv[u][2] = xg[l2];
         }
-        {
-            const uint32_t r = t / COBS;
-            cv = r < live_rows ? a.co[size_t(n0) * COBS + t] : 0.0f;  // 512 = 16 rows x 32
-        }
-        tv[0] = t < AT ? a.actor[L::B1 + t] : 0.0f;
-        tv[1] = t < 2 * HID + 1 ? a.critic[C_B1 + t] : 0.0f;
-        if (t < live_rows) {  // the row's objective inputs, used after the layers
-            const uint32_t mrow = n0 + t;
+        cv = a.co[size_t(n0) * COBS + (t / COBS < live_rows ? t : t % COBS)];  // 512 = 16 rows x 32
+        tv[0] = a.actor[L::B1 + (t < AT ? t : 0)];
+        tv[1] = a.critic[C_B1 + (t < 2 * HID + 1 ? t : 0)];
+        if (wv == 2) {  // the rows' objective inputs, used after the layers
+            const uint32_t mrow = n0 + (l < live_rows ? l : 0);
 #pragma unroll
             for (uint32_t q = 0; q < 4; q++) ract[q] = a.actions[size_t(mrow) * 4 + q];
             rolp = a.old_logp[mrow];
             radv = a.adv[mrow];  // normalised where it is used, so no load waits on it here
             rret = a.ret[mrow];
+            if (a.norm) { nmean = a.norm[0]; ninv = a.norm[1]; }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        const uint32_t p0 = mb_pos(l), p1 = p0 + 64, p2 = mb_pos(l + 128);
+        float* ws = s_w + wv * NU * MB_WS;
+#pragma unroll
+        for (uint32_t u = 0; u < NU; u++) {
+            ws[u * MB_WS + p0] = w[u][0];
+            ws[u * MB_WS + p1] = w[u][1];
+            if (l < MB_KP - 128) ws[u * MB_WS + p2] = last ? w[u][2] : -0.0f;
         }
 #pragma unroll
-        for (uint32_t k = 0; k < NW; k++) {
-            const uint32_t e = t + 512 * k;
-            if (e < D * HID) s_w[(e % D) * WS + e / D] = w[k];
-        }
+        for (uint32_t k = 0; k < 4; k++) s_cw[(t / COBS + 16 * k) * MB_CS + mb_pos(t % COBS)] = cw[k];
+        float* xs = s_x + wv * NR * MB_WS;
 #pragma unroll
-        for (uint32_t k = 0; k < NCW; k++) {
-            const uint32_t e = t + 512 * k;
-            s_cw[(e % COBS) * WS + e / COBS] = cw[k];
+        for (uint32_t u = 0; u < NR; u++) {
+            const bool in = wv * NR + u < live_rows;
+            xs[u * MB_WS + p0] = in ? xv[u][0] : 0.0f;
+            xs[u * MB_WS + p1] = in ? xv[u][1] : 0.0f;
+            if (l < MB_KP - 128) xs[u * MB_WS + p2] = in && last ? xv[u][2] : 0.0f;
         }
-#pragma unroll
-        for (uint32_t k = 0; k < NX; k++) {
-            const uint32_t e = t + 512 * k;
-            if (e < MB_FWD_ROWS * D) s_x[e / D][e % D] = xv[k];
-        }
-        s_c[t / COBS][t % COBS] = cv;
-        if (t < AT) s_at[t] = tv[0];
-        if (t < 2 * HID + 1) s_ct[t] = tv[1];
+        s_c[(t / COBS) * MB_CS + mb_pos(t % COBS)] = t / COBS < live_rows ? cv : 0.0f;
+        if (t < AT) s_t[t] = tv[0];
+        if (t < 2 * HID + 1) s_t[AT + t] = tv[1];
     }
-    static_assert(MB_FWD_ROWS * COBS == 512 && COBS * HID % 512 == 0 && 5 * HID + 8 <= 512, "staging map");
     __syncthreads();
+    // First layers.  The hidden values take the place of the wavefront's own
+    // 16 weight rows, which no other reads: unit 16 g + c of row r at
+    // 16 g * stride + 20 r + c (s_w: actor, s_cw: critic).
+    constexpr uint32_t HA = 16 * MB_WS, HC = 16 * MB_CS;
     {
         const bool actor = wv < 4;
-        const uint32_t unit = 16 * (wv % 4) + l % 16;
+        const uint32_t g = wv % 4, c = l % 16, q = l / 16, unit = 16 * g + c;
         const float bias = actor ? s_at[unit] : s_ct[unit];
         v4f acc = {bias, bias, bias, bias};
         if (actor) {
-            constexpr uint32_t NK = (D + 3) / 4;
-#pragma unroll 8
-            for (uint32_t st = 0; st < NK; st++) {
-                const uint32_t k = 4 * st + l / 16;
-                const float av = k < D ? s_x[l % 16][k] : 0.0f;
-                const float bv = k < D ? s_w[k * WS + unit] : -0.0f;
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av, bv, acc, 0, 0, 0);
+            const float* xr = s_x + c * MB_WS;
+            const float* wr = s_w + unit * MB_WS;
+#pragma unroll
+            for (uint32_t j = 0; j < 11; j++) {
+                const v4f av = *reinterpret_cast<const v4f*>(xr + 16 * j + 4 * q);
+                const v4f bv = *reinterpret_cast<const v4f*>(wr + 16 * j + 4 * q);
+#pragma unroll
+                for (uint32_t s = 0; s < 4; s++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[s], bv[s], acc, 0, 0, 0);
             }
+            const v2f av = *reinterpret_cast<const v2f*>(xr + 176 + 2 * q);
+            const v2f bv = *reinterpret_cast<const v2f*>(wr + 176 + 2 * q);
+#pragma unroll
+            for (uint32_t s = 0; s < 2; s++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[s], bv[s], acc, 0, 0, 0);
         } else {
 #pragma unroll
-            for (uint32_t st = 0; st < COBS / 4; st++) {
-                const uint32_t k = 4 * st + l / 16;
-                acc = __builtin_amdgcn_mfma_f32_16x16x4f32(s_c[l % 16][k], s_cw[k * WS + unit], acc, 0, 0, 0);
+            for (uint32_t j = 0; j < COBS / 16; j++) {
+                const v4f av = *reinterpret_cast<const v4f*>(s_c + c * MB_CS + 16 * j + 4 * q);
+                const v4f bv = *reinterpret_cast<const v4f*>(s_cw + unit * MB_CS + 16 * j + 4 * q);
+#pragma unroll
+                for (uint32_t s = 0; s < 4; s++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(av[s], bv[s], acc, 0, 0, 0);
             }
         }
+        float* hs = actor ? s_w + g * HA : s_cw + g * HC;
 #pragma unroll
-        for (uint32_t r = 0; r < 4; r++) {
-            const float h = tanh_f(acc[r]);
-            if (actor) s_ha[4 * (l / 16) + r][unit] = h;
-            else s_hc[4 * (l / 16) + r][unit] = h;
-        }
+        for (uint32_t r = 0; r < 4; r++) hs[MB_HS * (4 * q + r) + c] = tanh_f(acc[r]);
+        // the row scale factors, beside the actor's longer chain
+        if (t >= 256 && t < 264) s_ex[t - 256] = row_scale_exp(s_at + 5 * HID + 4, t - 256);
     }
     __syncthreads();
     const float* w2 = s_at + HID;          // actor W2 [4][64]
     const float* cw2 = s_ct + HID;         // critic w2 [64]
-    if (t < 4 * MB_FWD_ROWS) {  // means (ppo.hpp:73-78)
+    if (wv == 0) {  // means (ppo.hpp:73-78): lane 4 r + q
         const uint32_t r = t / 4, q = t % 4;
         float z = s_at[5 * HID + q];
-        for (uint32_t k = 0; k < HID; k++) z = fma_f(w2[q * HID + k], s_ha[r][k], z);
-        if (D == MDN_ACTOR_OBS_PRIOR && q < 3) z += s_x[r][D - 3 + q];
+        v4f hv[HID / 4], wq[HID / 4];
+#pragma unroll
+        for (uint32_t k = 0; k < HID / 4; k++) {
+            hv[k] = *reinterpret_cast<const v4f*>(s_w + (k / 4) * HA + MB_HS * r + 4 * (k % 4));
+            wq[k] = *reinterpret_cast<const v4f*>(w2 + q * HID + 4 * k);
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < HID; k++) z = fma_f(wq[k / 4][k % 4], hv[k / 4][k % 4], z);
+        if (D == MDN_ACTOR_OBS_PRIOR && q < 3) z += s_x[r * MB_WS + mb_pos(D - 3 + q)];
         s_mv[r][q] = z;
-    } else if (t < 5 * MB_FWD_ROWS) {  // value (ppo.hpp:82-93)
-        const uint32_t r = t - 4 * MB_FWD_ROWS;
+    } else if (t >= 64 && t < 64 + MB_FWD_ROWS) {  // value (ppo.hpp:82-93)
+        const uint32_t r = t - 64;
         float v = s_ct[2 * HID];
-        for (uint32_t k = 0; k < HID; k++) v = fma_f(cw2[k], s_hc[r][k], v);
+        v4f hv[HID / 4], wq[HID / 4];
+#pragma unroll
+        for (uint32_t k = 0; k < HID / 4; k++) {
+            hv[k] = *reinterpret_cast<const v4f*>(s_cw + (k / 4) * HC + MB_HS * r + 4 * (k % 4));
+            wq[k] = *reinterpret_cast<const v4f*>(cw2 + 4 * k);
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < HID; k++) v = fma_f(wq[k / 4][k % 4], hv[k / 4][k % 4], v);
         s_mv[r][4] = v;
-    } else if (t < 5 * MB_FWD_ROWS + 8) {
-        s_ex[t - 5 * MB_FWD_ROWS] = row_scale_exp(s_at + 5 * HID + 4, t - 5 * MB_FWD_ROWS);
+    }
+    // Wavefronts 4-7 write the row records, four units of a row per thread;
+    // what does not need the objective before it is known.
+    const uint32_t dr = (t % 256) / 16, dk = 4 * (t % 16);
+    const size_t row = (ONE ? n0 : n0 % CHUNK) + dr;
+    v4f ga = {0.0f, 0.0f, 0.0f, 0.0f}, gc = ga, cwv = ga, wq[4] = {ga, ga, ga, ga};
+    if (wv >= 4) {
+        const v4f ha = *reinterpret_cast<const v4f*>(s_w + (dk / 16) * HA + MB_HS * dr + dk % 16);
+        const v4f hc = *reinterpret_cast<const v4f*>(s_cw + (dk / 16) * HC + MB_HS * dr + dk % 16);
+        *reinterpret_cast<v4f*>(rec + MB_HA + row * HID + dk) = ha;
+        *reinterpret_cast<v4f*>(rec + MB_HC + row * HID + dk) = hc;
+#pragma unroll
+        for (uint32_t q = 0; q < 4; q++) wq[q] = *reinterpret_cast<const v4f*>(w2 + q * HID + dk);
+        cwv = *reinterpret_cast<const v4f*>(cw2 + dk);
+#pragma unroll
+        for (uint32_t u = 0; u < 4; u++) {
+            ga[u] = 1.0f - ha[u] * ha[u];
+            gc[u] = 1.0f - hc[u] * hc[u];
+        }
+    }
+    // Wavefront 2, idle meanwhile, has what the objective needs beside them in
+    // registers.
+    float ls[4] = {0.0f, 0.0f, 0.0f, 0.0f}, ex[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}, adv = 0.0f;
+    const float scale = 1.0f / max_f(float(a.b), 1.0f);
+    if (wv == 2) {
+#pragma unroll
+        for (uint32_t q = 0; q < 4; q++) ls[q] = s_at[5 * HID + 4 + q];
+#pragma unroll
+        for (uint32_t q = 0; q < 8; q++) ex[q] = s_ex[q];
+        adv = a.norm ? (radv - nmean) * ninv : radv;
+        if (a.norm && l < live_rows) a.adv_out[n0 + l] = adv;
     }
     __syncthreads();
-    const float scale = 1.0f / max_f(float(a.b), 1.0f);
-    if (t < MB_FWD_ROWS) {
-        float* rs = s_rs[t];
-        if (t < live_rows) {
-            const uint32_t mrow = n0 + t;
-            const float mean[4] = {s_mv[t][0], s_mv[t][1], s_mv[t][2], s_mv[t][3]};
-            const float value = s_mv[t][4], target = rret;
+    if (wv == 2 && l < MB_FWD_ROWS) {
+        float* rs = s_rs[l];
+        if (l < live_rows) {
+            const float mean[4] = {s_mv[l][0], s_mv[l][1], s_mv[l][2], s_mv[l][3]};
+            const float value = s_mv[l][4], target = rret;
             float dmean[4];
-            const float adv = normalized_advantage(a, radv);
-            if (a.norm) a.adv_out[mrow] = adv;
-            row_objective(a, s_at + 5 * HID + 4, s_ex, ract, rolp, adv, mean, value, target, scale, dmean, rs);
+            row_objective(a, ls, ex, ract, rolp, adv, mean, value, target, scale, dmean, rs);
             rs[12] = a.vcoef * (value - target) * scale;
         } else {
             for (uint32_t c = 0; c < 13; c++) rs[c] = 0.0f;
         }
     }
     __syncthreads();
-    {   // hidden deltas (ppo.metal:470-485, 618-631) and the row records
-        const uint32_t r = t / 32, k0 = t % 32;
-        const bool live = r < live_rows;
-        const size_t row = (ONE ? n0 : n0 % CHUNK) + r;
+    if (wv >= 4) {   // hidden deltas (ppo.metal:470-485, 618-631)
+        const bool live = dr < live_rows;
+        const v4f dm = *reinterpret_cast<const v4f*>(s_rs[dr]);
+        const float dv = s_rs[dr][12];
+        v4f da, dc;
 #pragma unroll
-        for (uint32_t u = 0; u < 2; u++) {
-            const uint32_t k = k0 + 32 * u;
+        for (uint32_t u = 0; u < 4; u++) {
             float d = 0.0f;
 #pragma unroll
-            for (uint32_t q = 0; q < 4; q++) d = fma_f(s_rs[r][q], w2[q * HID + k], d);
-            const float ha = s_ha[r][k], hc = s_hc[r][k];
-            rec[MB_HA + row * HID + k] = ha;
-            rec[MB_DA + row * HID + k] = live ? d * (1.0f - ha * ha) : 0.0f;
-            rec[MB_HC + row * HID + k] = hc;
-            rec[MB_DC + row * HID + k] = live ? s_rs[r][12] * cw2[k] * (1.0f - hc * hc) : 0.0f;
+            for (uint32_t q = 0; q < 4; q++) d = fma_f(dm[q], wq[q][u], d);
+            da[u] = live ? d * ga[u] : 0.0f;
+            dc[u] = live ? dv * cwv[u] * gc[u] : 0.0f;
         }
-        if (k0 < 16) rec[MB_RS + row * 16 + k0] = s_rs[r][k0];
+        *reinterpret_cast<v4f*>(rec + MB_DA + row * HID + dk) = da;
+        *reinterpret_cast<v4f*>(rec + MB_DC + row * HID + dk) = dc;
+        rec[MB_RS + row * 16 + t % 16] = s_rs[dr][t % 16];
     }
 }
 
@@ -1270,12 +1346,12 @@ __global__ __launch_bounds__(512) void mb_forward_kernel(MbArgs m) {
 // actor inputs ceil((D+1)/16) x 4 unit blocks, critic 3 x 4, actor row
 // scalars 5 (h blocks 0-3 and the ones column), critic row scalars 4.
 //
-// The operands' way from memory bounds a tile, not its 64 matrix-core steps
-// (0.9 us): one wavefront has 128 loads to issue, two round trips at 63 in
+// The operands' way from memory bounds a tile more than its 64 matrix-core
+// steps: one wavefront has 128 loads to issue, two round trips at 63 in
 // flight.  Four wavefronts load 64 rows each at once and run their part of
 // the chain in turn, the accumulator passing through LDS.  A 256-row
 // minibatch: 6.2 -> 4.6 us (eight wavefronts of 32 rows: 4.8 us, more
-// passing); 16 chunks of 256 rows: the step 2 % faster.
+// passing); at 16 chunks of 256 rows the step is 2 % faster.
 constexpr uint32_t MB_GRAD_WAVES = 4;
 template <uint32_t D>
 constexpr uint32_t mb_actor_in_tiles() { return (D + 1 + 15) / 16; }
