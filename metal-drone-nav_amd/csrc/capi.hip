@@ -1379,7 +1379,10 @@ struct MdnLargePPO {
     mdn::PolicyShape shape;
     float *actor = nullptr, *critic = nullptr, *am = nullptr, *av = nullptr, *cm = nullptr, *cv = nullptr;
     __bf16 *awb = nullptr, *cwb = nullptr;
-    __bf16 *xa = nullptr, *xaT = nullptr, *xc = nullptr, *xcT = nullptr;  // bf16 rows of one minibatch
+    // bf16 rows: `prepared` minibatches (the first is also the forward-only
+    // calls' buffer)
+    __bf16 *xa = nullptr, *xaT = nullptr, *xc = nullptr, *xcT = nullptr;
+    uint32_t prepared = 1;
     float* eval_means = nullptr;                         // [rows][4]
     float* fwd_part = nullptr;                           // forward partial sums over hidden slices
     float *means = nullptr, *values = nullptr, *dm = nullptr, *dls = nullptr, *dv = nullptr, *loss = nullptr;
@@ -1478,6 +1481,9 @@ void mdn_lppo_destroy(MdnLargePPO* p) {
     delete p;
 }
 
+// Most bytes of prepared rows a wide trainer keeps (896 a row).
+static constexpr size_t LP_PREP_BYTES = size_t(4) << 30;
+
 int mdn_lppo_create(MdnSim* s, uint32_t hidden, uint32_t epochs, uint32_t minibatch, MdnLargePPO** out) {
     if (!s || !out) return fail(MDN_E_ARG, "mdn_lppo_create: null argument");
     *out = nullptr;
@@ -1504,11 +1510,20 @@ int mdn_lppo_create(MdnSim* s, uint32_t hidden, uint32_t epochs, uint32_t miniba
     guard(dev_alloc(&p->cv, C));
     guard(dev_alloc(&p->awb, size_t(hidden) * 192));
     guard(dev_alloc(&p->cwb, size_t(hidden) * 32));
-    const size_t MP = (M + 127) / 128 * 128;
-    guard(dev_alloc(&p->xa, MP * 192));
-    guard(dev_alloc(&p->xaT, MP * 192));
-    guard(dev_alloc(&p->xc, MP * 32));
-    guard(dev_alloc(&p->xcT, MP * 32));
+    // With several epochs every minibatch keeps its bf16 rows through the
+    // update, prepared in the first epoch only (20 us per 32,768-row minibatch
+    // of about 400), while they take at most LP_PREP_BYTES and the device has
+    // twice their size free; otherwise one minibatch's buffers serve in turn.
+    const size_t MP = (M + 127) / 128 * 128, bytes = MP * 2 * (192 + 32) * sizeof(__bf16);
+    const size_t batches = p->updates / epochs;
+    size_t free_bytes = 0, total_bytes = 0;
+    if (epochs > 1 && batches * bytes <= LP_PREP_BYTES && hipMemGetInfo(&free_bytes, &total_bytes) == hipSuccess &&
+        free_bytes / 2 >= batches * bytes)
+        p->prepared = uint32_t(batches);
+    guard(dev_alloc(&p->xa, p->prepared * MP * 192));
+    guard(dev_alloc(&p->xaT, p->prepared * MP * 192));
+    guard(dev_alloc(&p->xc, p->prepared * MP * 32));
+    guard(dev_alloc(&p->xcT, p->prepared * MP * 32));
     guard(dev_alloc(&p->eval_means, R * 4));
     guard(dev_alloc(&p->nv_count, 1));
     guard(dev_alloc(&p->nv_idx, R));
@@ -1637,15 +1652,23 @@ int mdn_lppo_rollout_update(MdnLargePPO* p, uint32_t rollout_index) {
     const std::vector<uint32_t> order = mdn::minibatch_schedule(rows, p->minibatch, p->epochs, rollout_index);
     if (order.size() != p->updates) return fail(MDN_E_STATE, "wide PPO update count mismatch");
     const uint32_t H = p->hidden, D = p->shape.obs;
+    const size_t MP = (size_t(p->minibatch) + 127) / 128 * 128;
+    std::vector<uint8_t> ready(p->prepared, 0);  // minibatches prepared by this update
     for (size_t u = 0; u < order.size(); u++) {
         const uint32_t begin = order[u];
+        const size_t slot = p->prepared > 1 ? begin / p->minibatch : 0;
+        __bf16 *xa = p->xa + slot * MP * 192, *xaT = p->xaT + slot * MP * 192;
+        __bf16 *xc = p->xc + slot * MP * 32, *xcT = p->xcT + slot * MP * 32;
         const uint32_t b = std::min(p->minibatch, rows - begin);
         const float* obs = s->obs + size_t(begin) * D;
         const float* co = s->co + size_t(begin) * COBS;
         rc = timed(s, MDN_K_LP_FORWARD, [&] {
-            hipError_t e = lp_launch_prep(obs, co, b, D, p->xa, p->xaT, p->xc, p->xcT, true, s->stream);
+            hipError_t e = hipSuccess;
+            if (p->prepared == 1 && p->updates > p->epochs || !ready[slot])
+                e = lp_launch_prep(obs, co, b, D, xa, xaT, xc, xcT, true, s->stream);
+            ready[slot] = 1;
             if (e == hipSuccess)
-                e = lp_launch_forward(p->xa, p->xc, p->awb, p->cwb, p->actor, p->critic, H, D, b, lp_prior(p, obs),
+                e = lp_launch_forward(xa, xc, p->awb, p->cwb, p->actor, p->critic, H, D, b, lp_prior(p, obs),
                                       p->means, p->values, p->fwd_part, s->stream);
             if (e == hipSuccess)
                 e = lp_launch_loss(p->means, p->values, s->actions + size_t(begin) * 4, s->logp + begin,
@@ -1656,7 +1679,7 @@ int mdn_lppo_rollout_update(MdnLargePPO* p, uint32_t rollout_index) {
         });
         if (rc) return rc;
         rc = timed(s, MDN_K_LP_BACKWARD, [&] {
-            return lp_launch_backward(p->xa, p->xaT, p->xc, p->xcT, p->awb, p->cwb, p->actor, p->critic, p->dm, p->dv,
+            return lp_launch_backward(xa, xaT, xc, xcT, p->awb, p->cwb, p->actor, p->critic, p->dm, p->dv,
                                       p->col_part, H, D, b, p->part, p->ga, p->gc, p->scratch, s->stream);
         });
         if (rc) return rc;

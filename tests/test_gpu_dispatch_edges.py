@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 
 from gpu_compare import ENV_BUFFERS, ROW_BUFFERS, compare, config, make_pair
-from mdnav import native, ops, task_runtime, task_settings
+from mdnav import LargePPOTrainer, Sim, native, ops, task_runtime, task_settings
 from oracle_lib import oracle, ptr
 
 pytestmark = pytest.mark.gpu
@@ -172,6 +172,38 @@ def test_normalize_sizes(count):
         assert hip.hipFree(dev) == 0
         assert np.array_equal(host[offset:offset + count], want), offset
         assert np.all(host[:offset] == 7.0) and np.all(host[offset + count:] == 7.0)
+
+
+def _order(rows, minibatch, epochs, rollout):
+    out = np.zeros(-(-rows // minibatch) * epochs, np.uint32)
+    oracle().orc_minibatch_schedule(rows, minibatch, epochs, rollout, ptr(out))
+    return out.tolist()
+
+
+@pytest.mark.parametrize("hidden", [128, 384])
+@pytest.mark.parametrize("n,minibatch", [(50, 500), (50, 260), (61, 200)])
+def test_wide_epochs(n, minibatch, hidden):
+    """The wide update keeps its prepared rows from the first epoch on: three
+    epochs equal three one-epoch updates in the same orders bit for bit (one
+    minibatch, two and four, ragged last ones), and so does a second update on
+    other rows."""
+    say("case: wide update of", n, "x 10 rows, minibatches of", minibatch, "hidden", hidden)
+    T, epochs = 10, 3
+    cfg = config(n=n, family=1, seed=7, max_steps=6)
+    sims = [Sim(cfg, T, actor_obs=184) for _ in range(2)]
+    a, b = LargePPOTrainer(sims[0], hidden, epochs, minibatch), LargePPOTrainer(sims[1], hidden, 1, minibatch)
+    per = -(-n * T // minibatch)
+    for rollout in range(2):
+        a.collect()
+        b.collect()
+        a.rollout_update(rollout)
+        order = _order(n * T, minibatch, epochs, rollout)
+        for e in range(epochs):
+            want = order[per * e:per * (e + 1)]
+            b.rollout_update(next(r for r in range(10000) if _order(n * T, minibatch, 1, r) == want))
+        assert a.optimizer_step == b.optimizer_step == per * epochs * (rollout + 1)
+        for name in ("actor", "critic", "actor_m", "actor_v", "critic_m", "critic_v"):
+            assert np.array_equal(a.get(name), b.get(name)), (rollout, name)
 
 
 def _mlp(d, h, b, seed, special):
