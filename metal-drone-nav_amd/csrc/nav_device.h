@@ -946,10 +946,14 @@ __device__ __forceinline__ void derivative(const MdnPhysicsParams& P, const Phys
 // only the sign of a zero may differ, and the derivative has no operation -
 // a division by a computed value, a sign test - that turns the sign of a zero
 // into a difference of value).  Those values reach the state only as addends
-// of state components, so when no state component is -0 (no_negative_zero)
+// of state components, so when no state component is -0 (quad_state)
 // every stage state and the next state are bit-identical: s + (+-0) is s for
-// s != 0 and +0 for s = +0.  wm = wind / mass, formed once per tick with the
-// same division.
+// s != 0 and +0 for s = +0.  A zero drops its term only beside a finite factor
+// (0 * inf is NaN), so every value here must be finite as well.  That holds for
+// the Crazyflie plant and a state within QUAD_RANGE; with any other plant an
+// infinite or NaN value leaves the next state so before its limits,
+// physics_step<true> reports it and the step is taken again with derivative().
+// wm = wind / mass, formed once per tick with the same division.
 __device__ __forceinline__ void derivative_quad(const MdnPhysicsParams& P, const PhysRecip& RP, const State& s,
                                                 const float sp[4], const float wm[3], State& d) {
     float m[4];
@@ -1001,15 +1005,68 @@ __device__ __forceinline__ void derivative_quad(const MdnPhysicsParams& P, const
     }
 }
 
-// true when no component of s is -0 (the condition derivative_quad needs;
-// a physics step keeps it, since a sum is -0 only when both addends are)
-__device__ __forceinline__ bool no_negative_zero(const State& s) {
+// What the components of a state look like, in integer form: the largest
+// exponent field (kNotFinite for an infinity or NaN) and the smallest bits with
+// the sign turned (0 for a -0).
+constexpr uint32_t kNotFinite = 0x7f800000u;
+struct StateBits {
+    uint32_t exponent = 0u, zero = 0xffffffffu;
+};
+__device__ __forceinline__ StateBits state_bits(const State& s) {
     const float* a = &s.p[0];
-    bool ok = true;
+    StateBits b;
 #pragma unroll
-    for (int i = 0; i < 17; ++i) ok = ok && float_bits(a[i]) != 0x80000000u;
-    return ok;
+    for (int i = 0; i < 17; ++i) {
+        const uint32_t u = float_bits(a[i]);
+        b.exponent = max(b.exponent, u & kNotFinite);
+        b.zero = min(b.zero, u ^ 0x80000000u);
+    }
+    return b;
 }
+// The states from which no value of a standard-structure Crazyflie step can
+// overflow: every component below QUAD_RANGE, in metres, metres and radians a
+// second and rotor speeds alike (flight stays far below it).
+constexpr float QUAD_RANGE = 256.0f, QUAD_WIND = 1e30f;  // accelerations by wind: up to QUAD_WIND
+template <bool RANGE>
+__device__ __forceinline__ bool quad_state(const StateBits& b) {
+    return b.zero != 0u && (!RANGE || b.exponent < __builtin_bit_cast(uint32_t, QUAD_RANGE));
+}
+// The bound itself: the largest magnitude of any value of the four stages, from
+// the largest plant words and state components (each stage starts from the
+// state plus the last stage's derivative).
+constexpr double larger(double a, double b) { return a < b ? b : a; }
+constexpr double magnitude(double a) { return a < 0 ? -a : a; }
+constexpr double quad_step_bound(const MdnPhysicsParams& P) {
+    double c[3] = {0, 0, 0}, arm = 0, rate = 0, inertia = 0, inverse = 0, gravity = 0;
+    for (int r = 0; r < 4; ++r) {
+        for (int i = 0; i < 3; ++i) {
+            c[i] = larger(c[i], magnitude(P.rotor_thrust_coefficients[3 * r + i]));
+            arm = larger(arm, magnitude(P.rotor_positions[3 * r + i]));
+        }
+        arm = larger(arm, magnitude(P.rotor_torque_constants[r]));
+        rate = larger(rate, larger(1.0 / P.rotor_time_constants_rising[r], 1.0 / P.rotor_time_constants_falling[r]));
+    }
+    for (int i = 0; i < 9; ++i) {
+        inertia = larger(inertia, magnitude(P.inertia[i]));
+        inverse = larger(inverse, magnitude(P.inertia_inverse[i]));
+    }
+    for (int i = 0; i < 3; ++i) gravity = larger(gravity, magnitude(P.gravity_world[i]));
+    const double limit = larger(larger(magnitude(P.action_min), magnitude(P.action_max)), QUAD_RANGE);
+    double bound = 0, dr = 0, dw = 0, dq = 0;
+    for (int stage = 0; stage < 4; ++stage) {
+        const double h = stage == 0 ? 0.0 : stage == 3 ? P.dt : 0.5 * P.dt;
+        const double r = limit + h * dr, w = limit + h * dw, q = limit + h * dq;
+        const double m = c[0] + c[1] * r + c[2] * r * r, thrust = 4 * m * (1 + 8 * q * q), gyro = 2 * inertia * w * w;
+        dr = (limit + r) * rate;
+        dq = 3 * q * w;
+        dw = inverse * (4 * m * arm + gyro);
+        const double dv = thrust / P.mass + gravity + QUAD_WIND;
+        bound = larger(larger(larger(bound, thrust), larger(gyro, dr)), larger(larger(dq, dw), dv));
+    }
+    return bound;
+}
+// (16: the sums of stages and of state and stage)
+static_assert(16.0 * quad_step_bound(mdn::kCrazyflie) < 3.4e38, "a Crazyflie step from within QUAD_RANGE stays finite");
 
 __device__ __forceinline__ void axpy_state(const State& s, const State& d, float scale, State& out) {
     const float* a = &s.p[0];
@@ -1019,18 +1076,35 @@ __device__ __forceinline__ void axpy_state(const State& s, const State& d, float
     for (int i = 0; i < 17; ++i) o[i] = a[i] + scale * b[i];
 }
 
-// physics.hpp:122-179.  QUAD: the standard-structure derivative
-// (derivative_quad; `wind` is then wind / mass).
+// x limited to [-limit, limit] with the comparisons of physics.hpp:165-173,
+// which let NaN through (the median of three would drop it).
+__device__ __forceinline__ float limited(float x, float limit) {
+    const float y = __builtin_amdgcn_fmed3f(x, -limit, limit);
+    return x == x ? y : x;
+}
+// true when every component of s is finite (x * 0 is a zero, else NaN)
+__device__ __forceinline__ bool all_finite(const State& s) {
+    const float* a = &s.p[0];
+    float t[2] = {0.0f, 0.0f};  // two chains
+#pragma unroll
+    for (int i = 0; i < 17; ++i) t[i % 2] = fma_f(a[i], 0.0f, t[i % 2]);
+    return t[0] == t[1];
+}
+
+// physics.hpp:122-179.  Returns whether every component of the next state is
+// finite.  QUAD: the standard-structure derivative (derivative_quad; `wind` is
+// then wind / mass); a component then counts as it is before its limit, and a
+// step that is not finite holds no result.
 template <bool QUAD = false>
-__device__ __forceinline__ void physics_step(const MdnPhysicsParams& P, const PhysRecip& RP, const State& s,
+__device__ __forceinline__ bool physics_step(const MdnPhysicsParams& P, const PhysRecip& RP, const State& s,
                                              const float action[4], const float wind[3], State& next) {
     float sp[4];
     const float half = (P.action_max - P.action_min) * 0.5f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         // the clamps to nonzero bounds as a median of three: for a non-NaN
-        // value it is the comparisons' result, -0 included (a NaN state is
-        // rejected by the caller's validity check either way)
+        // value it is the comparisons' result, -0 included (RAPTOR's actions
+        // are clipped, never NaN)
         const float a = __builtin_amdgcn_fmed3f(action[i], -1.0f, 1.0f);
         sp[i] = a * half + P.action_min + half;
     }
@@ -1067,17 +1141,27 @@ __device__ __forceinline__ void physics_step(const MdnPhysicsParams& P, const Ph
     const double inv_norm = 1.0 / double(norm);
 #pragma unroll
     for (int i = 0; i < 4; ++i) next.q[i] = div_r(next.q[i], inv_norm);
+    bool finite = true;
+    if constexpr (QUAD) finite = all_finite(next);
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-        next.p[i] = __builtin_amdgcn_fmed3f(next.p[i], -P.position_limit, P.position_limit);
-        next.v[i] = __builtin_amdgcn_fmed3f(next.v[i], -P.velocity_limit, P.velocity_limit);
-        next.w[i] = __builtin_amdgcn_fmed3f(next.w[i], -P.angular_velocity_limit, P.angular_velocity_limit);
+        if constexpr (QUAD) {  // finite, or the result is not used
+            next.p[i] = __builtin_amdgcn_fmed3f(next.p[i], -P.position_limit, P.position_limit);
+            next.v[i] = __builtin_amdgcn_fmed3f(next.v[i], -P.velocity_limit, P.velocity_limit);
+            next.w[i] = __builtin_amdgcn_fmed3f(next.w[i], -P.angular_velocity_limit, P.angular_velocity_limit);
+        } else {
+            next.p[i] = limited(next.p[i], P.position_limit);
+            next.v[i] = limited(next.v[i], P.velocity_limit);
+            next.w[i] = limited(next.w[i], P.angular_velocity_limit);
+        }
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         if (next.rpm[i] < P.action_min) next.rpm[i] = P.action_min;
         if (next.rpm[i] > P.action_max) next.rpm[i] = P.action_max;
     }
+    if constexpr (!QUAD) finite = all_finite(next);
+    return finite;
 }
 
 // ---------------------------------------------------------------- world generation

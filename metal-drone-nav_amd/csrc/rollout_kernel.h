@@ -928,6 +928,25 @@ __global__ __launch_bounds__(64 * W) void rollout_kernel(RolloutArgs a) {
     bool deferred = false, prev_due = false;
     bool co_fresh = false;  // s_co holds this env's critic observation of its current state
     size_t prev_row = 0;
+    // derivative_quad's conditions on the env's state.  Fused kernels form them
+    // here and at a reset, each physics step keeps them, and between ticks they
+    // are in LDS (at 8,192 envs: carried in registers they cost 0.6 % of the
+    // rollout, the scalar registers being full, and formed anew every tick 1 %).
+    // RANGE: the Crazyflie's steps are kept finite by bounding the state.  The
+    // small fleets' launches of one tick retry instead, like other plants, which
+    // is 1 % faster there (and 0.5 % slower in the large fleets).  A wind beyond
+    // QUAD_WIND drives the velocity to its limit, beyond QUAD_RANGE, at every
+    // step.
+    constexpr bool RANGE = CF && !(S && SPLIT);
+    auto plain_state = [&] {
+        bool ok = quad_state<RANGE>(state_bits(s));
+        if constexpr (RANGE)
+#pragma unroll
+            for (int j = 0; j < 3; j++) ok = ok && __builtin_fabsf(world[166 + j]) <= QUAD_WIND;
+        return ok;
+    };
+    __shared__ uint32_t s_plain[SPLIT ? 1 : E];
+    if constexpr (!SPLIT) s_plain[grp] = plain_state();
     for (uint32_t t = 0; t < a.count; t++) {
         const uint32_t tick = SPLIT ? (a.tick0 + t) % a.horizon : t % a.horizon;
         const size_t row = size_t(tick) * N + nn;
@@ -1568,9 +1587,9 @@ __global__ __launch_bounds__(64 * W) void rollout_kernel(RolloutArgs a) {
         const float wind[3] = {world[166] * EP.mass, world[167] * EP.mass, world[168] * EP.mass};
         // the standard-structure derivative takes wind / mass, the same
         // division physics.hpp:101 repeats in every derivative evaluation
-        const double rmass = DYN ? s_erp[DYN ? grp : 0].mass : RP.mass;
-        const float wm[3] = {div_r(wind[0], rmass), div_r(wind[1], rmass), div_r(wind[2], rmass)};
-        bool nzero = no_negative_zero(s);  // no component of s is -0 (derivative_quad's condition)
+        const PhysRecip& ER = DYN ? s_erp[DYN ? grp : 0] : RP;
+        const float wm[3] = {div_r(wind[0], ER.mass), div_r(wind[1], ER.mass), div_r(wind[2], ER.mass)};
+        bool plain = SPLIT ? plain_state() : s_plain[SPLIT ? 0 : grp] != 0u;
         for (uint32_t step = 0; step < C.substeps; step++) {
             float mo[22] = {0};
             if (!done) {
@@ -1601,30 +1620,33 @@ __global__ __launch_bounds__(64 * W) void rollout_kernel(RolloutArgs a) {
 #pragma unroll
                 for (int q = 0; q < 4; q++) r.motors[q] = act[q];
                 State nx;
-                if constexpr (DYN) {
-                    if (plants_quad && !__any(!nzero)) physics_step<true>(EP, s_erp[grp], s, act, wm, nx);
-                    else physics_step(EP, s_erp[grp], s, act, wind, nx);
-                } else if ((CF || a.quad) && !__any(!nzero)) physics_step<true>(P, RP, s, act, wm, nx);
-                else physics_step(P, RP, s, act, wind, nx);
-                // every component finite (isfinite_f) and none -0, in integer
-                // form: the largest exponent field and the smallest bits ^ sign
-                const float* nf = &nx.p[0];
-                uint32_t emax = 0u, zmin = 0xffffffffu;
-#pragma unroll
-                for (int j = 0; j < 17; j++) {
-                    const uint32_t u = float_bits(nf[j]);
-                    emax = max(emax, u & 0x7f800000u);
-                    zmin = min(zmin, u ^ 0x80000000u);
+                // the standard-structure derivative where its conditions hold
+                // in the whole wavefront; RANGE keeps its step finite,
+                // otherwise one that is not is taken again in general form
+                bool valid;
+                if constexpr (RANGE) {
+                    if (__any(!plain)) physics_step(P, RP, s, act, wind, nx);
+                    else physics_step<true>(P, RP, s, act, wm, nx);
+                } else {
+                    bool quad = (DYN ? plants_quad : CF || a.quad) && !__any(!plain);
+                    if (quad) {
+                        valid = physics_step<true>(EP, ER, s, act, wm, nx);
+                        quad = !__any(!valid);
+                    }
+                    if (!quad) valid = physics_step(EP, ER, s, act, wind, nx);
                 }
-                const bool valid = emax != 0x7f800000u;
-                if (!valid) {
+                const StateBits nb = state_bits(nx);
+                if constexpr (RANGE) valid = nb.exponent != kNotFinite;
+                // (laying the usual case out first is worth 0.5 % to the large
+                // fleets and costs the fused small fleets 0.7 %)
+                if (S ? !valid : __builtin_expect(!valid, 0)) {
                     collision = true;
                     done = true;
                 } else {
                     const float ex = s.p[0] - nx.p[0], ey = s.p[1] - nx.p[1], ez = s.p[2] - nx.p[2];
                     r.path += sqrt_f(ex * ex + ey * ey + ez * ez);
                     s = nx;
-                    nzero = zmin != 0u;
+                    plain = quad_state<RANGE>(nb);
                     r.elapsed += P.dt;
                     const float cl = clearance(mk(s.p[0], s.p[1], s.p[2]), r.elapsed);
                     step_clearance = min_f(step_clearance, cl);
@@ -1637,6 +1659,8 @@ __global__ __launch_bounds__(64 * W) void rollout_kernel(RolloutArgs a) {
                 }
             }
         }
+
+        if constexpr (!SPLIT) s_plain[grp] = plain;
 
         // ---- outcome (sim.metal:304-306), next value, episode end
         bool ended = false;
@@ -1770,6 +1794,7 @@ __global__ __launch_bounds__(64 * W) void rollout_kernel(RolloutArgs a) {
         group_sync();
         if (ended) {  // sim_reset_one, not first
             reset_apply(C, P, RW, nn, false, reset_rng, world, s, r);
+            if constexpr (!SPLIT) s_plain[grp] = plain_state();
 #pragma unroll
             for (int j = 0; j < U; j++) hu[j] = RW[2000 + lane + G * j];
             if constexpr (W > 1)
