@@ -266,9 +266,10 @@ __global__ __launch_bounds__(64 * WAVES) void memory_hint_kernel(nav::MemoryArgs
                 // of |p|^2, radius^2, along^2 and their difference, below
                 // 5e-7 |p|^2 together; its value is at least along - radius
                 // (1 + 2^-22); and the fma chain differs from the exact along -
-                // radius by less than 5e-7 (1 + |p|).  The margin is several
-                // times these, and the root's own error.
-                const float margin = 2e-6f * (8.0f + p2), c2 = p2 - ly - margin;
+                // radius by less than 5e-7 (1 + |p| + radius).  The margin is
+                // several times these, and the root's own error.  (The radius
+                // counts with points minutes old: 0.15 m a second.)
+                const float margin = 2e-6f * (8.0f + p2 + radius), c2 = p2 - ly - margin;
                 const float c = (c2 > 0.0f ? __builtin_amdgcn_sqrtf(c2) * 0.999999f : 0.0f) - margin;
                 const float low = radius * 1.0001f + margin;
                 held[k] = make_float4(x, y, z, -low);

@@ -102,6 +102,38 @@ def test_memory_workgroups(n):
     _collect_both(sim, ora, 9)
 
 
+@pytest.mark.parametrize("dt", [0.05, 5.0, 500.0, 5e3, 5e5])
+def test_memory_point_radius(dt):
+    """Remembered points of every age: a point's sphere grows by 0.15 m a
+    second, so a slow sensor gives spheres of kilometres around points near
+    the body, and their contacts start at along = 0 to the last bit."""
+    say("case: geometry memory, sensor interval", dt)
+    n, period = 512, int(round(dt / 0.05))
+    cfg = config(n=n, family=1, seed=13, speed=1.0, distance=3.0, geometry_memory=1, sensor_period=period,
+                 max_steps=1 << 30)
+    sim, _, ora = make_pair(cfg, 1, actor_obs=184)
+    ora.set("actor", sim.get("actor"))
+    ora.set("critic", sim.get("critic"))
+    sim.reset()
+    ora.reset()
+    rng = np.random.default_rng(13)
+    runs, poses = sim.get("runs"), sim.get("poses").reshape(n, 8, 12)
+    runs["steps"] = 7 * period + (1 if period > 1 else 0)  # eight frames held, none due unless every tick has one
+    sensors = np.full((n, 8, 320), 12.0, np.float32)
+    frame, pixel = rng.integers(0, 7, n), rng.integers(0, 320, n)
+    sensors[np.arange(n), frame, pixel] = rng.uniform(0.011, 0.05, n)  # one hit per env, centimetres away
+    poses[:, :, :3] = sim.get("states")["position"][:, None] + rng.uniform(-0.03, 0.03, (n, 8, 3))
+    poses[:, :, 3:] = np.eye(3, dtype=np.float32).reshape(9)
+    for x in (sim, ora):
+        x.set("runs", runs)
+        x.set("sensors", sensors)
+        x.set("poses", poses)
+        x.collect(1)
+    sim.sync()
+    bad = compare(sim, ora, ENV_BUFFERS + ROW_BUFFERS)
+    assert not bad, bad
+
+
 @pytest.mark.parametrize("obs", [181, 184])
 @pytest.mark.parametrize("n,T,minibatch", [(257, 1, 257), (64, 8, 512), (100, 83, 4150), (2048, 10, 20480),
                                            (20481, 1, 20481)])
