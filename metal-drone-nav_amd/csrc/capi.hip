@@ -1379,8 +1379,8 @@ struct MdnLargePPO {
     mdn::PolicyShape shape;
     float *actor = nullptr, *critic = nullptr, *am = nullptr, *av = nullptr, *cm = nullptr, *cv = nullptr;
     __bf16 *awb = nullptr, *cwb = nullptr;
-    // bf16 rows: `prepared` minibatches (the first is also the forward-only
-    // calls' buffer)
+    // bf16 rows of `prepared` minibatches (1: every minibatch in turn; the
+    // first is also the forward-only calls' buffer)
     __bf16 *xa = nullptr, *xaT = nullptr, *xc = nullptr, *xcT = nullptr;
     uint32_t prepared = 1;
     float* eval_means = nullptr;                         // [rows][4]
@@ -1481,8 +1481,28 @@ void mdn_lppo_destroy(MdnLargePPO* p) {
     delete p;
 }
 
-// Most bytes of prepared rows a wide trainer keeps (896 a row).
+// Most bytes of prepared rows a wide trainer keeps (896 a row of a minibatch
+// padded to whole 128 rows).
 static constexpr size_t LP_PREP_BYTES = size_t(4) << 30;
+
+// bf16 row buffers for `minibatches` minibatches of MP padded rows; on failure
+// none is held.
+static int lp_alloc_rows(MdnLargePPO* p, size_t minibatches, size_t MP) {
+    int rc = dev_alloc(&p->xa, minibatches * MP * 192);
+    if (!rc) rc = dev_alloc(&p->xaT, minibatches * MP * 192);
+    if (!rc) rc = dev_alloc(&p->xc, minibatches * MP * 32);
+    if (!rc) rc = dev_alloc(&p->xcT, minibatches * MP * 32);
+    if (!rc) {
+        p->prepared = uint32_t(minibatches);
+        return MDN_OK;
+    }
+    for (__bf16** b : {&p->xa, &p->xaT, &p->xc, &p->xcT}) {
+        if (*b) hipFree(*b);
+        *b = nullptr;
+    }
+    (void)hipGetLastError();  // the next launch's check is not to report it
+    return rc;
+}
 
 int mdn_lppo_create(MdnSim* s, uint32_t hidden, uint32_t epochs, uint32_t minibatch, MdnLargePPO** out) {
     if (!s || !out) return fail(MDN_E_ARG, "mdn_lppo_create: null argument");
@@ -1510,20 +1530,6 @@ int mdn_lppo_create(MdnSim* s, uint32_t hidden, uint32_t epochs, uint32_t miniba
     guard(dev_alloc(&p->cv, C));
     guard(dev_alloc(&p->awb, size_t(hidden) * 192));
     guard(dev_alloc(&p->cwb, size_t(hidden) * 32));
-    // With several epochs every minibatch keeps its bf16 rows through the
-    // update, prepared in the first epoch only (20 us per 32,768-row minibatch
-    // of about 400), while they take at most LP_PREP_BYTES and the device has
-    // twice their size free; otherwise one minibatch's buffers serve in turn.
-    const size_t MP = (M + 127) / 128 * 128, bytes = MP * 2 * (192 + 32) * sizeof(__bf16);
-    const size_t batches = p->updates / epochs;
-    size_t free_bytes = 0, total_bytes = 0;
-    if (epochs > 1 && batches * bytes <= LP_PREP_BYTES && hipMemGetInfo(&free_bytes, &total_bytes) == hipSuccess &&
-        free_bytes / 2 >= batches * bytes)
-        p->prepared = uint32_t(batches);
-    guard(dev_alloc(&p->xa, p->prepared * MP * 192));
-    guard(dev_alloc(&p->xaT, p->prepared * MP * 192));
-    guard(dev_alloc(&p->xc, p->prepared * MP * 32));
-    guard(dev_alloc(&p->xcT, p->prepared * MP * 32));
     guard(dev_alloc(&p->eval_means, R * 4));
     guard(dev_alloc(&p->nv_count, 1));
     guard(dev_alloc(&p->nv_idx, R));
@@ -1546,6 +1552,23 @@ int mdn_lppo_create(MdnSim* s, uint32_t hidden, uint32_t epochs, uint32_t miniba
     guard(dev_alloc(&p->metric_rows, size_t(p->updates) * 4));
     guard(dev_alloc(&p->metric_mean, 4));
     guard(dev_alloc(&p->grad_norm_rows, size_t(p->updates) * 2));
+    // The row buffers come last, when what the trainer cannot do without is
+    // there.  With several epochs every minibatch keeps its bf16 rows through
+    // the update, prepared in the first epoch only (20 us per 32,768-row
+    // minibatch of about 400), while they take at most LP_PREP_BYTES, the
+    // padding no more than the rows themselves, and the device has twice their
+    // size free; otherwise, or if they cannot be had, one minibatch's buffers
+    // serve in turn.
+    if (rc == MDN_OK) {
+        const size_t MP = (M + 127) / 128 * 128, batches = p->updates / epochs;
+        const size_t bytes = batches * MP * 2 * (192 + 32) * sizeof(__bf16);
+        size_t free_bytes = 0, total_bytes = 0;
+        bool held = false;
+        if (epochs > 1 && batches > 1 && batches * MP <= 2 * R && bytes <= LP_PREP_BYTES &&
+            hipMemGetInfo(&free_bytes, &total_bytes) == hipSuccess && free_bytes / 2 >= bytes)
+            held = lp_alloc_rows(p, batches, MP) == MDN_OK;
+        if (!held) guard(lp_alloc_rows(p, 1, MP));
+    }
     if (rc == MDN_OK) {
         std::vector<float> a(A), c(C);
         mdn::init_policy(p->shape, a.data(), c.data());

@@ -238,6 +238,30 @@ def test_wide_epochs(n, minibatch, hidden):
             assert np.array_equal(a.get(name), b.get(name)), (rollout, name)
 
 
+@pytest.mark.parametrize("n,minibatch", [(20, 50), (5, 20), (13, 63), (24, 60)])
+def test_wide_epochs_in_turn(n, minibatch):
+    """The same with one minibatch's buffers serving every minibatch in turn:
+    rows whose padding to 128 would take more than they do are not kept."""
+    test_wide_epochs(n, minibatch, 128)
+
+
+def test_wide_small_minibatch_memory():
+    """Rows of tiny minibatches are not kept padded: 65,536 of them in pairs
+    would take 3.8 GB, the trainer's other buffers a few MB."""
+    from test_zz_no_alloc import hip_runtime
+    say("case: wide trainer, 65,536 rows in minibatches of 2")
+    hip = hip_runtime()
+    hip.hipMemGetInfo.argtypes = [ctypes.POINTER(ctypes.c_size_t)] * 2
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    sim = Sim(config(n=4096, family=1, seed=7), 16, actor_obs=184)
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    before = free.value
+    p = LargePPOTrainer(sim, 128, 3, 2)
+    assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    assert before - free.value < 256 << 20, before - free.value
+    p.close()
+
+
 def _mlp(d, h, b, seed, special):
     rng = np.random.default_rng(seed)
     w = rng.normal(0, 0.3, h * d + h + 4 * h + 8).astype(np.float32)
