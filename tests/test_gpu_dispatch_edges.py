@@ -277,6 +277,23 @@ def _mlp(d, h, b, seed, special):
     return w, x
 
 
+@pytest.mark.parametrize("d,h,b", [(3, 7, 5), (181, 64, 17), (184, 64, 16), (200, 130, 20)])
+def test_forward_subnormal_sums(d, h, b):
+    """Inputs and weights so small that every product, partial sum and
+    activation is subnormal: none is flushed to zero."""
+    say("case: forward,", b, "rows", d, "inputs", h, "units, subnormal sums")
+    w, x = _mlp(d, h, b, d, 0)
+    w[:h * d + h] *= np.float32(1e-20)
+    w[h * d:h * d + h] *= np.float32(1e-20)
+    x *= np.float32(1e-20)
+    ho, mo = np.zeros((b, h), np.float32), np.zeros((b, 4), np.float32)
+    oracle().orc_actor_forward_batch(ptr(w), ptr(x), d, h, b, ptr(ho), ptr(mo))
+    tiny = np.finfo(np.float32).tiny
+    assert np.all(np.abs(ho) < tiny) and np.count_nonzero(ho) > ho.size // 2
+    hid, mean = ops.actor_forward(w, x, hidden_dim=h)
+    assert np.array_equal(hid, ho) and np.array_equal(mean, mo)
+
+
 @pytest.mark.parametrize("special", [0, 1])
 @pytest.mark.parametrize("d,h,b", [(1, 1, 1), (2, 5, 3), (4, 64, 16), (181, 64, 17), (184, 63, 33), (191, 65, 15),
                                    (193, 128, 31), (192, 256, 16), (385, 257, 20), (824, 320, 18), (1024, 512, 1)])
