@@ -86,7 +86,7 @@ struct MdnSim {
     uint32_t* run = nullptr;
     float* world = nullptr;
     float* sensors = nullptr;
-    float* pool_ring = nullptr;  // [N][8][80]
+    float* pool_ring = nullptr;  // [N][8][80] (fleets above nav::SMALL_FLEET)
     float* poses = nullptr;
     float* commands = nullptr;
     float* raptor = nullptr;
@@ -326,7 +326,7 @@ int mdn_sim_create(const MdnSimConfig* cfg, uint32_t horizon, const MdnRaptorWei
     guard(dev_alloc(&s->run, size_t(RUN_WORDS) * N));
     guard(dev_alloc(&s->world, size_t(WORLD_WORDS) * N));
     guard(dev_alloc(&s->sensors, size_t(N) * 8 * 320));
-    guard(dev_alloc(&s->pool_ring, size_t(N) * 8 * 80));
+    if (N > nav::SMALL_FLEET) guard(dev_alloc(&s->pool_ring, size_t(N) * 8 * 80));
     guard(dev_alloc(&s->poses, size_t(N) * 96));
     guard(dev_alloc(&s->commands, size_t(N) * 32));
     guard(dev_alloc(&s->raptor, 2084));

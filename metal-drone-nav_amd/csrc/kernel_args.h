@@ -14,8 +14,9 @@ struct RolloutArgs {
     float* world;          // [N][169]
     float* sensors;        // [N][8][320]
     // pooled 2x2 minima of the last K frames, slot f % K ([N][K][80]): the
-    // ring the four-wavefront kernels with K > 2 keep in HBM (their LDS has
-    // no room for it); rebuilt from `sensors` at every launch
+    // ring the 32-env kernels with K > 2 keep in HBM (their LDS has no room
+    // for it); rebuilt from `sensors` at every launch, null for fleets that
+    // those kernels do not take
     float* pool_ring;
     float* poses;          // [N][8][12]
     float* commands;       // [N][8][4]
@@ -157,7 +158,6 @@ struct RowArgs {
     uint32_t d;             // actor inputs: 181, or 184 with the geometry-prior hint
 };
 
-// cpu_reference.hpp:553-567 inputs for one update of both networks.
 // A minibatch of few 256-row gradient chunks split over many workgroups: the
 // row-parallel forward writes per-row records to `rec`, the
 // parameter-parallel pass writes the finished gradient to `grad` (one chunk)
@@ -175,6 +175,7 @@ constexpr uint32_t MB_REC_WORDS = 4 * 256 * 64 + 256 * 16;
 constexpr uint32_t MB_MAX_CHUNKS = 80;
 constexpr uint32_t CHUNK_ROWS = 256;  // rows of one gradient chunk
 
+// cpu_reference.hpp:553-567 inputs for one update of both networks.
 struct AdamArgs {
     float* actor; float* critic; float* actor_w1t; float* critic_w1t;
     float* am; float* av; float* cm; float* cv;

@@ -180,9 +180,9 @@ hipError_t nav_launch_reset(const nav::RolloutArgs* a, hipStream_t stream) {
 // Lanes per env G and pooled ring slots K are compile-time; K = sensor_delay+2
 // rounded up to 2, 4 or 8.
 // The 8-lane cases run four wavefronts per workgroup with the weights in LDS
-// (32 envs, one workgroup per CU); with 4 or 8 slots the pooled ring lives
-// in HBM (a.pool_ring).  16 and 4 lanes per env run one wavefront per
-// workgroup with the weights in L1/L2.
+// (32 envs, one workgroup per CU); with 4 or 8 slots the pooled ring lives in
+// HBM (a.pool_ring), except in the small-fleet instances.  16 and 4 lanes per
+// env run one wavefront per workgroup with the weights in L1/L2.
 // Split ticks (a->ext_means set) and 184-input actors are built for 8 lanes
 // per env only.
 // 8-lane fleets of at most nav::SMALL_FLEET envs, and every launch with

@@ -547,7 +547,7 @@ static_assert(offsetof(MdnPhysicsParams, rotor_thrust_directions) == 48 &&
 // W = wavefronts per workgroup.  W == 1: weights and camera rays are read from
 // global memory (L1/L2 resident).  W > 1: the workgroup stages one copy of the
 // actor first layer, the RAPTOR weights and the camera rays in LDS, shared by
-// its 64*W/G envs.
+// its envs (64*W/G; small fleets 4*epw).
 // Tails of the flat policy vectors (ppo.hpp:35-45) from the first bias on:
 // actor b1[HID], W2[4][HID], b2[4], log_std[4]; critic b1[HID], W2[HID], b2.
 constexpr uint32_t ACTOR_TAIL = 5 * HID + 8, CRITIC_TAIL = 2 * HID + 1;
@@ -597,6 +597,7 @@ struct WeightLds<1, D, V> {};
 template <int G, int K, int W, bool X, uint32_t D, bool DYN, bool CF = false, bool S = false>
 __global__ __launch_bounds__(64 * W) void rollout_kernel(RolloutArgs a) {
     static_assert(!S || (W == 4 && G == 8), "small fleets: four wavefronts, 8 lanes per env");
+    static_assert(W > 1 || (D == MDN_ACTOR_OBS_POOLED && !X && !DYN), "one wavefront: the fused 181-input rollout");
     constexpr int E = S ? 16 : 64 * W / G;    // env rows in LDS
     constexpr int U = 16 / G;        // RAPTOR units per lane
     constexpr int HU = 64 / G;       // actor/critic hidden units per lane
@@ -1459,7 +1460,6 @@ __global__ __launch_bounds__(64 * W) void rollout_kernel(RolloutArgs a) {
                     float z = A[a_b2 + q];
 #pragma unroll 8
                     for (uint32_t h = 0; h < HID; h++) z = fma_f(A[a_w2 + q * HID + h], s_ah[grp][h], z);
-                    if (D == MDN_ACTOR_OBS_PRIOR && q < 3) z += s_obs[grp][D - 3 + q];  // ppo.hpp:77
                     mean[q] = z;
                 }
                 value = CR[c_b2];
@@ -1736,7 +1736,7 @@ __global__ __launch_bounds__(64 * W) void rollout_kernel(RolloutArgs a) {
         co_fresh = active && !ended;
         if constexpr (X) {
             // next values are the caller's (from the stored next critic observations)
-        } else if constexpr (W > 1) {  // next value: critic hidden of s' for all 32 envs
+        } else if constexpr (W > 1) {  // next value: critic hidden of s' for every env of the workgroup
             wg_reset = __syncthreads_or(ended) != 0;
             // with no reset in the workgroup and another tick to come in this
             // launch, the next tick's critic at s forms these next values
